@@ -113,10 +113,11 @@ int jinf_hip_engine_n_past(const jinf_hip_engine* e);
 int jinf_hip_engine_forward(jinf_hip_engine* e, const int32_t* tokens, int n_tokens,
                             const float** logits);
 
-/* Decodes a prompt of n_tokens tokens in steps of up to 64 tokens, every GEMV
- * running on a step's tokens at once on the matrix cores (the batched path
- * of jinf_hip_batch_prefill, over this engine's own cache) and token i
- * attending to the positions up to its own.  Leaves the engine where
+/* Decodes a prompt of n_tokens tokens in steps of many tokens (up to 1024;
+ * 64 or fewer in one batched step), every projection running on a step's
+ * tokens at once on the matrix cores (the path of jinf_hip_batch_prefill,
+ * over this engine's own cache) and token i attending to the positions up to
+ * its own.  Leaves the engine where
  * jinf_hip_engine_forward on the same tokens would (position advanced by
  * n_tokens, next token the last token's argmax, *logits the last token's
  * logits); per token the arithmetic is that loop's, with the batched GEMVs'
@@ -199,14 +200,14 @@ int  jinf_hip_batch_n_past(const jinf_hip_batch* b, int seq);
  * [-1, n_vocab) or a token for a sequence whose context is full. */
 int  jinf_hip_batch_forward(jinf_hip_batch* b, const int32_t* tokens, const float** logits);
 
-/* Prompt of sequence seq: decodes its n_tokens ids (each in [0, n_vocab))
- * in chunks of up to n_seq tokens per step, every GEMV running on a chunk's
- * tokens at once and token i attending to the sequence's positions up to its
- * own, so the sequence ends where n_tokens forward steps of its own would
+/* Prompt of sequence seq: decodes its n_tokens ids (each in [0, n_vocab)),
+ * every projection running on a step's tokens at once (up to n_seq tokens in
+ * a batched step; longer prompts in steps of up to 1024) and token i
+ * attending to the sequence's positions up to its own, so the sequence ends where n_tokens forward steps of its own would
  * leave it (position advanced by n_tokens, next token the last token's
- * argmax); other sequences are untouched.  The last chunk's per-token logits
- * occupy rows 0 .. m - 1 of the batch's logits (the last token's at row
- * (n_tokens - 1) mod n_seq); *logits (may be NULL) receives the device
+ * argmax); other sequences are untouched.  The logits of the prompt's last
+ * m = (n_tokens - 1) mod n_seq + 1 tokens occupy rows 0 .. m - 1 of the
+ * batch's logits; *logits (may be NULL) receives the device
  * pointer of that row.  Status 5 when the prompt does not fit the sequence's
  * context or an id is outside [0, n_vocab).  The reference feeds a prompt
  * one token at a time (src/engine.cpp:684-760); per token the arithmetic is

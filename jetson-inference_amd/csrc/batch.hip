@@ -17,6 +17,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <new>
 #include <vector>
 
@@ -25,6 +26,7 @@
 #include "jinf_device.h"
 #include "jinf_host.h"
 #include "matvec_batch_internal.h"
+#include "prefill_internal.h"
 #include "quant_device.h"
 
 namespace jinf {
@@ -177,6 +179,14 @@ struct jinf_hip_batch {
     size_t aws_bytes = 0;
     int32_t* h_io = nullptr;  // pinned: n_seq tokens, 16 words, 3 n_seq prefill row words
     std::vector<int> h_pos;   // host copy of the positions
+    // the wide prompt path's buffers, made on the first prompt long enough
+    // (wide_state 1; -1: not available, prompts take steps of n_seq rows)
+    int wide_state = 0;
+    char* wide = nullptr;
+    PfBuf pf;
+    float *w_hidden = nullptr, *w_q = nullptr, *w_attn = nullptr, *w_ff = nullptr, *w_up = nullptr;
+    int32_t* w_rows = nullptr;    // [3][pf.rows] tokens, positions, lengths
+    int32_t* h_wide = nullptr;    // the same, pinned
     hipStream_t stream = nullptr;
     // captured steps, one per attention bound (a power of two >= 64, at most
     // max_ctx): the bound sets the attention's launch geometry and covers
@@ -188,17 +198,17 @@ struct jinf_hip_batch {
 
 namespace {
 
-int bat_embed(jinf_hip_batch* b, int rows) {
+int bat_embed(jinf_hip_batch* b, float* hidden, const int32_t* ids, int rows) {
     const jinf_hip_engine_desc& d = *b->d;
     const dim3 grid((d.n_embd + 255) / 256, rows);
     if (d.token_embd_type == JINF_HIP_F32)
-        return launch(bat_embed_dense_kernel<float>, grid, dim3(256), 0, b->stream, b->hidden,
-                      static_cast<const float*>(d.token_embd), b->acts, d.n_vocab, d.n_embd);
+        return launch(bat_embed_dense_kernel<float>, grid, dim3(256), 0, b->stream, hidden,
+                      static_cast<const float*>(d.token_embd), ids, d.n_vocab, d.n_embd);
     if (d.token_embd_type == JINF_HIP_F16)
-        return launch(bat_embed_dense_kernel<uint16_t>, grid, dim3(256), 0, b->stream, b->hidden,
-                      static_cast<const uint16_t*>(d.token_embd), b->acts, d.n_vocab, d.n_embd);
-    return jinf_dequant_rows(b->hidden, d.n_embd, d.token_embd, d.token_embd_type, d.n_vocab,
-                             d.n_embd, b->acts, rows, JINF_HIP_F32, b->stream);
+        return launch(bat_embed_dense_kernel<uint16_t>, grid, dim3(256), 0, b->stream, hidden,
+                      static_cast<const uint16_t*>(d.token_embd), ids, d.n_vocab, d.n_embd);
+    return jinf_dequant_rows(hidden, d.n_embd, d.token_embd, d.token_embd_type, d.n_vocab,
+                             d.n_embd, ids, rows, JINF_HIP_F32, b->stream);
 }
 
 // `pend`: the previous layer's deferred down-projection residual add, merged
@@ -219,13 +229,25 @@ int bat_qkv(jinf_hip_batch* b, const jinf_hip_layer_weights& w, void* kc, void* 
     return JINF_HIP_OK;
 }
 
+// The argmax of logits row `rows` - 1, sequence seq's next token.
+int bat_prefill_end(jinf_hip_batch* b, int rows, int seq, int new_pos) {
+    const int V = b->d->n_vocab;
+    const float* last = b->logits + (int64_t)(rows - 1) * V;
+    BAT_TRY(launch(bat_argmax_part_kernel, dim3(b->arg_parts, 1), dim3(kArgThreads), 0, b->stream,
+                   last, V, b->part_v, b->part_i));
+    return launch(bat_prefill_end_kernel, dim3(1), dim3(kArgThreads), 0, b->stream, last, V,
+                  b->part_v, b->part_i, b->arg_parts, b->pos + seq, b->cur + seq, new_pos);
+}
+
 // One step (src/engine.cpp:692-749 per row) over `rows` rows.  seq < 0: a
 // decode step, row s = sequence s (every sequence; tokens and positions from
 // the begin kernel).  seq >= 0: a prefill chunk, row i = prompt token i of
 // sequence seq (tokens, positions and lengths already in the row arrays);
 // the rows share the sequence's KV region (row stride 0), each writes its
-// own position's K / V rows and attends up to them.
-int bat_enqueue_rows(jinf_hip_batch* b, int rows, int seq, int new_pos) {
+// own position's K / V rows and attends up to them.  Only the prompt's last
+// chunk has logits anybody reads: without `head` the step ends after the
+// layers.
+int bat_enqueue_rows(jinf_hip_batch* b, int rows, int seq, int new_pos, bool head = true) {
     const jinf_hip_engine_desc& d = *b->d;
     hipStream_t s = b->stream;
     const int n = d.n_embd, nff = d.n_ff, ns = rows;
@@ -237,7 +259,7 @@ int bat_enqueue_rows(jinf_hip_batch* b, int rows, int seq, int new_pos) {
         BAT_TRY(launch(bat_begin_kernel, dim3((ns + 255) / 256), dim3(256), 0, s, b->st, b->htok,
                        b->cur, b->pos, b->acts, b->positions, b->lens, b->hist, b->hist_rows, ns,
                        b->max_ctx));
-    BAT_TRY(bat_embed(b, ns));
+    BAT_TRY(bat_embed(b, b->hidden, b->acts, ns));
     // The output and down projections' residual adds are deferred: their
     // column-split partial sums are added into the residual stream by a merge
     // launch ahead of the next GEMV's preparation, so the GEMVs need no
@@ -281,20 +303,131 @@ int bat_enqueue_rows(jinf_hip_batch* b, int rows, int seq, int new_pos) {
                                        b->dpart, b->dpart_bytes, b->mws, b->mws_bytes, &pend,
                                        false, s));
     }
+    if (!head) return JINF_HIP_OK;
     BAT_TRY(rmsnorm_matvec_batch_m(d.output, d.output_type, b->hidden, n, d.output_norm,
                                    d.output_norm_type, eps, b->logits, d.n_vocab, d.n_vocab, n, ns,
                                    b->mws, b->mws_bytes, &pend, s));
-    if (prefill) {
-        const float* last = b->logits + (int64_t)(ns - 1) * d.n_vocab;
-        BAT_TRY(launch(bat_argmax_part_kernel, dim3(b->arg_parts, 1), dim3(kArgThreads), 0, s,
-                       last, d.n_vocab, b->part_v, b->part_i));
-        return launch(bat_prefill_end_kernel, dim3(1), dim3(kArgThreads), 0, s, last, d.n_vocab,
-                      b->part_v, b->part_i, b->arg_parts, b->pos + seq, b->cur + seq, new_pos);
-    }
+    if (prefill) return bat_prefill_end(b, ns, seq, new_pos);
     BAT_TRY(launch(bat_argmax_part_kernel, dim3(b->arg_parts, ns), dim3(kArgThreads), 0, s,
                    b->logits, d.n_vocab, b->part_v, b->part_i));
     return launch(bat_argmax_end_kernel, dim3(ns), dim3(kArgThreads), 0, s, b->logits, d.n_vocab,
                   b->part_v, b->part_i, b->arg_parts, b->st, b->acts, b->pos, b->cur);
+}
+
+void bat_wide_release(jinf_hip_batch* b) {
+    if (b->h_wide) (void)hipHostFree(b->h_wide);
+    if (b->wide) (void)hipFree(b->wide);
+    b->h_wide = nullptr;
+    b->wide = nullptr;
+}
+
+// The wide prompt path's buffers: up to kPfMaxRows tokens.
+int bat_wide_create(jinf_hip_batch* b) {
+    const jinf_hip_engine_desc& d = *b->d;
+    const int R = std::min(kPfMaxRows, (b->max_ctx + kPfTile - 1) / kPfTile * kPfTile);
+    const size_t n = d.n_embd, nff = d.n_ff, rows = R;
+    bool split_ffn = false;
+    for (int L = 0; L < d.n_layers; ++L)
+        split_ffn |= d.layers[L].ffn_gate_type != d.layers[L].ffn_up_type;
+    size_t off = 0;
+    auto take_b = [&](size_t bytes) {
+        const size_t o = off;
+        off = up256(off + bytes);
+        return o;
+    };
+    const size_t o_hidden = take_b(rows * n * 4), o_q = take_b(rows * b->q_dim * 4);
+    const size_t o_attn = take_b(rows * b->q_dim * 4), o_ff = take_b(rows * nff * 4);
+    const size_t o_up = take_b(split_ffn ? rows * nff * 4 : 0);
+    const size_t o_rec = take_b(pf_rec_bytes(R, (int)std::max(n, nff)));
+    const size_t o_inv = take_b(rows * 4), o_scale = take_b(rows * 8);
+    const size_t o_cs = take_b(rows * (size_t)b->head_dim / 2 * 8);
+    const size_t o_part = take_b(pf_part_bytes()), o_rows = take_b(3 * rows * 4);
+    BAT_TRY(hip_rc(hipMalloc((void**)&b->wide, off), "hipMalloc"));
+    BAT_TRY(hip_rc(hipHostMalloc((void**)&b->h_wide, 3 * rows * 4, hipHostMallocDefault),
+                   "hipHostMalloc"));
+    auto f = [&](size_t o) { return reinterpret_cast<float*>(b->wide + o); };
+    b->w_hidden = f(o_hidden);
+    b->w_q = f(o_q);
+    b->w_attn = f(o_attn);
+    b->w_ff = f(o_ff);
+    b->w_up = f(o_up);
+    b->w_rows = reinterpret_cast<int32_t*>(b->wide + o_rows);
+    b->pf.rows = R;
+    b->pf.rec = reinterpret_cast<uint8_t*>(b->wide + o_rec);
+    b->pf.inv_s = f(o_inv);
+    b->pf.scale = reinterpret_cast<float2*>(b->wide + o_scale);
+    b->pf.cs = reinterpret_cast<float2*>(b->wide + o_cs);
+    b->pf.part = f(o_part);
+    b->pf.part_bytes = pf_part_bytes();
+    return JINF_HIP_OK;
+}
+
+// T prompt tokens of sequence seq at once (T <= pf.rows), each projection one
+// matrix product over all of them; the rows (tokens, positions, lengths) are
+// in w_rows.  head_rows > 0: the last head_rows tokens' logits into logits
+// rows 0 .. head_rows - 1, and the last one's argmax.
+int bat_enqueue_wide(jinf_hip_batch* b, int T, int seq, int new_pos, int head_rows) {
+    const jinf_hip_engine_desc& d = *b->d;
+    hipStream_t s = b->stream;
+    const int n = d.n_embd, nff = d.n_ff, qd = b->q_dim;
+    const float eps = d.rms_norm_eps;
+    const size_t kv_off = (size_t)seq * b->max_ctx * b->kv_dim * b->kv_es;
+    const int32_t *ids = b->w_rows, *pos = ids + b->pf.rows, *lens = pos + b->pf.rows;
+    BAT_TRY(bat_embed(b, b->w_hidden, ids, T));
+    BAT_TRY(pf_rope_table(b->pf, pos, T, b->head_dim, d.rope_freq_base, s));
+    PfPend pend;
+    for (int L = 0; L < d.n_layers; ++L) {
+        const jinf_hip_layer_weights& w = d.layers[L];
+        char* kc = b->kv + (size_t)L * b->kv_layer_bytes + kv_off;
+        char* vc = b->kv + (size_t)(d.n_layers + L) * b->kv_layer_bytes + kv_off;
+        BAT_TRY(pf_prepare(b->pf, b->w_hidden, n, T, n, w.attn_norm, w.attn_norm_type, eps, &pend, s));
+        const void* W[3] = {w.attn_q, w.attn_k, w.attn_v};
+        const int types[3] = {w.attn_q_type, w.attn_k_type, w.attn_v_type};
+        bool done[3] = {false, false, false};
+        for (int i = 0; i < 3; ++i) {
+            if (done[i]) continue;
+            const void* p[3] = {nullptr, nullptr, nullptr};
+            for (int k = i; k < 3; ++k)
+                if (!done[k] && types[k] == types[i]) {
+                    p[k] = W[k];
+                    done[k] = true;
+                }
+            BAT_TRY(pf_qkv(b->pf, p[0], p[1], p[2], types[i], T, n, b->w_q, qd, kc, vc, b->kv_type,
+                           pos, b->max_ctx, b->head_dim, d.n_heads, d.n_heads_kv, s));
+        }
+        bool done_attn = false;
+        BAT_TRY(pf_attention(b->w_attn, qd, b->w_q, qd, kc, vc, b->kv_type, b->kv_dim, lens, T,
+                             b->bound, b->head_dim, d.n_heads, d.n_heads_kv, s, &done_attn));
+        if (!done_attn)
+            BAT_TRY(attention_decode_xrec(b->w_attn, qd, b->w_q, qd, kc, vc, b->kv_type, b->kv_dim,
+                                          0, lens, T, b->bound, b->head_dim, d.n_heads,
+                                          d.n_heads_kv, 0.0f, nullptr, 0, nullptr, s));
+        BAT_TRY(pf_prepare(b->pf, b->w_attn, qd, T, qd, nullptr, 0, 0.0f, nullptr, s));
+        BAT_TRY(pf_matmul(b->pf, w.attn_output, w.attn_output_type, T, n, qd, b->w_hidden, n, true,
+                          &pend, s));
+        BAT_TRY(pf_prepare(b->pf, b->w_hidden, n, T, n, w.ffn_norm, w.ffn_norm_type, eps, &pend, s));
+        if (w.ffn_gate_type == w.ffn_up_type) {
+            BAT_TRY(pf_swiglu(b->pf, w.ffn_gate, w.ffn_up, w.ffn_gate_type, T, nff, n, b->w_ff, nff,
+                              s));
+        } else {
+            BAT_TRY(pf_matmul(b->pf, w.ffn_gate, w.ffn_gate_type, T, nff, n, b->w_ff, nff, false,
+                              nullptr, s));
+            BAT_TRY(pf_matmul(b->pf, w.ffn_up, w.ffn_up_type, T, nff, n, b->w_up, nff, false,
+                              nullptr, s));
+            BAT_TRY(jinf_swiglu_rows(b->w_ff, nff, b->w_ff, nff, b->w_up, nff, T, nff,
+                                     JINF_HIP_F32, s));
+        }
+        BAT_TRY(pf_prepare(b->pf, b->w_ff, nff, T, nff, nullptr, 0, 0.0f, nullptr, s));
+        BAT_TRY(pf_matmul(b->pf, w.ffn_down, w.ffn_down_type, T, n, nff, b->w_hidden, n, true,
+                          &pend, s));
+    }
+    if (head_rows <= 0) return JINF_HIP_OK;
+    BAT_TRY(pf_merge(b->pf, b->w_hidden, n, T, n, &pend, s));
+    BAT_TRY(rmsnorm_matvec_batch_m(d.output, d.output_type,
+                                   b->w_hidden + (int64_t)(T - head_rows) * n, n, d.output_norm,
+                                   d.output_norm_type, eps, b->logits, d.n_vocab, d.n_vocab, n,
+                                   head_rows, b->mws, b->mws_bytes, nullptr, s));
+    return bat_prefill_end(b, head_rows, seq, new_pos);
 }
 
 int bat_enqueue_step(jinf_hip_batch* b) { return bat_enqueue_rows(b, b->n_seq, -1, 0); }
@@ -344,6 +477,7 @@ void bat_release(jinf_hip_batch* b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     for (const auto& g : b->graphs) (void)hipGraphExecDestroy(g.second);
     if (b->h_io) (void)hipHostFree(b->h_io);
+    bat_wide_release(b);
     if (b->kv && b->kv_owned) (void)hipFree(b->kv);
     if (b->act) (void)hipFree(b->act);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -589,29 +723,43 @@ extern "C" int jinf_hip_batch_prefill(jinf_hip_batch* b, int seq, const int32_t*
                  n_tokens, seq, p0, b->max_ctx);
         return JINF_HIP_ERR_INVALID;
     }
+    // Prompts longer than one batched step run wide: chunks of a multiple of
+    // n_seq tokens, so that the last chunk holds the rows whose logits the
+    // caller sees (of a borrowed cache only the last row's).
+    if (n_tokens > b->n_seq && b->wide_state == 0) {
+        b->wide_state = bat_wide_create(b) == JINF_HIP_OK ? 1 : -1;
+        if (b->wide_state < 0) bat_wide_release(b);
+    }
+    const int step = b->wide_state == 1 ? b->pf.rows / b->n_seq * b->n_seq : 0;
     int32_t* rw = b->h_io + b->n_seq + 16;  // tokens, positions, lengths of a chunk
     int last = 0;
-    for (int c = 0; c < n_tokens; c += b->n_seq) {
-        const int m = n_tokens - c < b->n_seq ? n_tokens - c : b->n_seq;
+    for (int c = 0; c < n_tokens;) {
+        const int left = n_tokens - c;
+        const bool wide = step > 0 && left > b->n_seq;
+        const int m = std::min(left, wide ? step : b->n_seq);
+        const bool final_chunk = m == left;
+        const int ld = wide ? b->pf.rows : b->n_seq;
+        int32_t* hr = wide ? b->h_wide : rw;
         for (int i = 0; i < m; ++i) {
-            rw[i] = tokens[c + i];
-            rw[b->n_seq + i] = p0 + c + i;
-            rw[2 * b->n_seq + i] = p0 + c + i + 1;
+            hr[i] = tokens[c + i];
+            hr[ld + i] = p0 + c + i;
+            hr[2 * ld + i] = p0 + c + i + 1;
         }
-        BAT_TRY(hip_rc(hipMemcpyAsync(b->acts, rw, (size_t)m * 4, hipMemcpyHostToDevice,
-                                      b->stream), "hipMemcpyAsync"));
-        BAT_TRY(hip_rc(hipMemcpyAsync(b->positions, rw + b->n_seq, (size_t)m * 4,
-                                      hipMemcpyHostToDevice, b->stream), "hipMemcpyAsync"));
-        BAT_TRY(hip_rc(hipMemcpyAsync(b->lens, rw + 2 * b->n_seq, (size_t)m * 4,
-                                      hipMemcpyHostToDevice, b->stream), "hipMemcpyAsync"));
+        int32_t* dst[3] = {b->acts, b->positions, b->lens};
+        for (int k = 0; k < 3; ++k)
+            BAT_TRY(hip_rc(hipMemcpyAsync(wide ? b->w_rows + k * ld : dst[k], hr + k * ld,
+                                          (size_t)m * 4, hipMemcpyHostToDevice, b->stream),
+                           "hipMemcpyAsync"));
         b->bound = bat_bound(b, p0 + c + m);
-        const int rc = bat_enqueue_rows(b, m, seq, p0 + c + m);
+        last = !wide ? m - 1 : b->kv_owned ? (n_tokens - 1) % b->n_seq : 0;
+        const int rc = wide ? bat_enqueue_wide(b, m, seq, p0 + c + m, final_chunk ? last + 1 : 0)
+                            : bat_enqueue_rows(b, m, seq, p0 + c + m, final_chunk);
         // the pinned rows are rewritten for the next chunk: wait for this one
         const int sc = hip_rc(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
         if (rc != JINF_HIP_OK) return rc;
         if (sc != JINF_HIP_OK) return sc;
         b->h_pos[seq] = p0 + c + m;
-        last = m - 1;
+        c += m;
     }
     if (logits) *logits = b->logits + (int64_t)last * d.n_vocab;
     return JINF_HIP_OK;

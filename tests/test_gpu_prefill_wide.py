@@ -1,0 +1,130 @@
+"""Prompts longer than a batched step (the wide path: matrix products over
+128-token tiles, attention over tiles of rows) against the oracle's
+token-by-token loop.
+
+Bars as for the engine's other paths, relative to the logit scale: 1e-4 with
+an fp32 cache (fp32 sums), 4e-4 with an fp16 cache (a cached value may round
+to its other fp16 neighbour).
+"""
+import numpy as np
+import pytest
+
+import jinf_amd
+import model_util as mu
+import oracle
+from oracle import engine as oeng
+
+pytestmark = pytest.mark.gpu
+
+F32, F16 = oracle.F32, oracle.F16
+Q4_0, Q8_0, Q4_K, Q6_K = oracle.Q4_0, oracle.Q8_0, oracle.Q4_K, oracle.Q6_K
+MATS = ("attn_q", "attn_k", "attn_v", "attn_output", "ffn_gate", "ffn_up", "ffn_down")
+
+
+def tokens(n, vocab, seed):
+    return [int(x) for x in np.random.default_rng(seed).integers(3, vocab, size=n)]
+
+
+def check(got, want, kv, what):
+    err = float(np.max(np.abs(got.astype(np.float64) - want)))
+    bar = (4e-4 if kv == F16 else 1e-4) * float(np.max(np.abs(want)))
+    assert err <= bar, f"{what}: {err:.3e} > {bar:.3e}"
+
+
+def decode(ref, toks):
+    for t in toks:
+        out = ref.step(t)
+    return out
+
+
+# One token past a batched step, the edges of a 128-token tile and of its
+# 32-token parts; every weight format alone and mixed within a layer; each
+# head size the attention kernel takes and one it does not.
+@pytest.mark.parametrize("n,types,heads,kv", [
+    (65, Q4_0, (8, 2), F16),
+    (127, Q8_0, (4, 4), F16),
+    (128, Q4_K, (8, 1), F32),
+    (129, Q6_K, (8, 4), F16),
+    (161, mu.MIXED, (4, 2), F16),
+    (300, mu.MIXED, (16, 2), F32),
+])
+def test_engine_prefill(n, types, heads, kv):
+    t = types if isinstance(types, dict) else {m: types for m in MATS}
+    hp, W = mu.tiny_model(seed=n, n_embd=512, n_heads=heads[0], n_heads_kv=heads[1], n_ff=768,
+                          n_vocab=301, types=t)
+    toks = tokens(n + 3, 301, n)
+    ref = oeng.Decoder(hp, W, max_context=n + 8, kv_type=kv)
+    with jinf_amd.Engine(hp, mu.to_device(W), n + 8, kv) as e:
+        e.prefill(toks[:n])
+        check(e.logits(), decode(ref, toks[:n]), kv, f"prompt of {n}")
+        assert e.n_past == n
+        # the cache rows and the position: decoding goes on from there
+        e.forward(toks[n:])
+        check(e.logits(), decode(ref, toks[n:]), kv, "after the prompt")
+
+
+def test_two_chunks_and_a_later_prompt():
+    """A prompt of two wide chunks, then another at a position inside the
+    context (an attention tile starting past its first row)."""
+    hp, W = mu.tiny_model(seed=5, n_layers=1, n_vocab=301)
+    toks = tokens(1250, 301, 5)
+    ref = oeng.Decoder(hp, W, max_context=1300, kv_type=F16)
+    with jinf_amd.Engine(hp, mu.to_device(W), 1300, F16) as e:
+        e.prefill(toks[:1100])
+        check(e.logits(), decode(ref, toks[:1100]), F16, "1100 tokens")
+        e.prefill(toks[1100:])
+        check(e.logits(), decode(ref, toks[1100:]), F16, "150 more")
+
+
+@pytest.mark.parametrize("n_seq,n", [(1, 40), (3, 131), (50, 120)])
+def test_batch_prefill_logits_rows(n_seq, n):
+    """The batch's rows after a wide prompt: the last chunk of n_seq tokens'
+    logits at rows 0 .. (n - 1) % n_seq, and no other sequence touched."""
+    hp, W = mu.tiny_model(seed=9, n_vocab=301)
+    toks = tokens(n, 301, n)
+    ref = oeng.Decoder(hp, W, max_context=160, kv_type=F16)
+    want = [ref.step(t) for t in toks]
+    with jinf_amd.Engine(hp, mu.to_device(W), 8, F16) as e, \
+            jinf_amd.Batch(e, n_seq, 160, F16) as b:
+        other = (n_seq - 1) if n_seq > 1 else None
+        if other is not None:
+            b.prefill(other, toks[:2])
+        b.prefill(0, toks)
+        rows = (n - 1) % n_seq + 1
+        got = b.logits()
+        for i in range(rows):
+            check(got[i], want[n - rows + i], F16, f"row {i}")
+        assert b.n_past(0) == n
+        if other is not None:
+            assert b.n_past(other) == 2
+            r2 = oeng.Decoder(hp, W, max_context=160, kv_type=F16)
+            for t in toks[:2]:
+                r2.step(t)
+            step = [-1] * n_seq
+            step[other] = toks[2]
+            b.forward(step)
+            check(b.logits()[other], r2.step(toks[2]), F16, "the other sequence")
+
+
+def test_nonfinite_token_leaves_earlier_rows_alone():
+    """A token whose K and V rows are not finite changes no earlier token's
+    logits (their attention does not reach it); its own are NaN."""
+    hp, W = mu.tiny_model(seed=11, n_vocab=301, embd_type=F32)
+    n, n_seq, at = 40, 16, 37
+    toks = tokens(n, 300, 11)
+    toks[at] = 300
+    for value in (np.nan, np.inf):
+        W["token_embd.weight"][0][300] = 0.0
+        W["token_embd.weight"][0][300, 5] = value
+        ref = oeng.Decoder(hp, W, max_context=64, kv_type=F16)
+        want = [ref.step(t) for t in toks[:at]]
+        with jinf_amd.Engine(hp, mu.to_device(W), 8, F16) as e, \
+                jinf_amd.Batch(e, n_seq, 64, F16) as b:
+            b.prefill(0, toks)
+            got = b.logits()
+            first = n - 8  # rows 0 .. 7 are tokens 32 .. 39
+            for i in range(8):
+                if first + i < at:
+                    check(got[i], want[first + i], F16, f"row {i}")
+                elif first + i == at:
+                    assert np.all(np.isnan(got[i])), f"row {i}"
