@@ -277,9 +277,9 @@ int jinf_dequant_rows(void* out, int ld_out, const void* table, int qtype, int n
  * device array of n_seq int32.  Fast path: head_dim 64 or 128, caches, q
  * and strides 16-byte aligned; an fp16 cache then runs on the matrix cores
  * (|q * scale| < 65504).  Nothing is allocated.  workspace (device memory,
- * optional: NULL or too small runs every sequence in one work item) lets an
- * fp16-cache call split long contexts (chunks of at least 256 positions)
- * over several workgroups, which merge their partial results themselves; it
+ * optional: NULL or too small runs every sequence in one work item) lets a
+ * call split long contexts (chunks of at least 256 positions) over several
+ * workgroups, which merge their partial results themselves; it
  * needs jinf_attention_workspace_bytes(n_seq, n_heads, head_dim, max_ctx)
  * bytes, zero-filled before its first use (every call leaves its merge
  * counters at zero again, so it is reused without clearing), and must not be

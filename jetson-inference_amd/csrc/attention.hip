@@ -12,36 +12,21 @@
 //
 // Design.  Decode attention streams the K and V rows once (2 * head_dim *
 // bytes per position and kv head) and is HBM-bound.  A workgroup owns one
-// (sequence, kv head) and the G query heads that read it, so each K/V byte is
-// fetched once for the whole GQA group; its waves split the positions into
-// 64-position tiles and keep flash-decoding state (running max m, sum l and
-// the output accumulator) in registers.  An fp16 cache runs on the matrix
-// cores (attn_mfma_kernel below); an fp32 cache (the reference's drop-in) on
-// the vector ALUs:
-//   - scores: LPP lanes per position, each with head_dim / LPP dims of every
-//     query head in registers (LPP chosen so that G * head_dim / LPP <= 64
-//     registers), load their slice of the K row (the row is read coalesced)
-//     and reduce the partial dots across the LPP lanes; the score goes to LDS;
-//   - softmax: lane t takes position t of the tile: one tile max and one sum
-//     per head (DPP wave reductions), one exp per position and head, and the
-//     probabilities go back to LDS;
-//   - P V: lane l owns dims l, l + 64, ... of every head; each V row is read
-//     coalesced once and multiplied into all G heads with probabilities read
-//     from LDS as broadcasts;
-//   - the waves' states merge through LDS at the end (flash-decoding combine,
-//     in wave order).
-// When there are too few (sequence, kv head) pairs to fill the GPU (batch-1
-// decode), each workgroup takes a single query head instead (the G heads of
-// a group then share the K/V bytes through L2) and gets up to 16 waves.
-// The reference's interface has no workspace, so the positions of one head
-// are not split across workgroups.
+// (sequence, kv head) and query heads that read it, so each K/V byte is
+// fetched once for the group; its waves split the positions into tiles and
+// keep flash-decoding state (running max m, sum l and the output accumulator)
+// in registers, merged through LDS at the end in wave order.  Long contexts
+// are split over workgroups when the caller gives a workspace.  An fp16 cache
+// runs on the matrix cores (attn_mfma_kernel below), an fp32 cache (the
+// reference's) on the vector ALUs (attention_f32.hip).
 //
-// head_dim 64 and 128 with 16-byte aligned rows take this kernel; anything
+// head_dim 64 and 128 with 16-byte aligned rows take these kernels; anything
 // else takes a one-wave-per-head kernel (dims on lanes, one wave reduction
 // per position) with the same arithmetic.
 #include <atomic>
 #include <mutex>
 
+#include "attention_device.h"
 #include "jinf_device.h"
 #include "jinf_host.h"
 #include "jinf/kernels.h"
@@ -60,183 +45,10 @@ template <> struct KV<uint16_t> {
     static __device__ __forceinline__ float get(const uint16_t* p, int i) { return h2f(p[i]); }
 };
 
-// n consecutive elements (n * sizeof(T) a multiple of 16, p 16-byte aligned)
-// widened to fp32.
-template <typename T, int N>
-__device__ __forceinline__ void load_row(const T* p, float (&f)[N]) {
-    if constexpr (sizeof(T) == 4) {
-        static_assert(N % 4 == 0, "fp32 slices are whole 16-byte chunks");
-#pragma unroll
-        for (int c = 0; c < N / 4; ++c) {
-            const float4 v = reinterpret_cast<const float4*>(p)[c];
-            f[4 * c] = v.x; f[4 * c + 1] = v.y; f[4 * c + 2] = v.z; f[4 * c + 3] = v.w;
-        }
-    } else {
-        static_assert(N % 8 == 0, "fp16 slices are whole 16-byte chunks");
-#pragma unroll
-        for (int c = 0; c < N / 8; ++c) {
-            const uint4 v = reinterpret_cast<const uint4*>(p)[c];
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                f[8 * c + 2 * i] = h2f((uint16_t)(w[i] & 0xFFFFu));
-                f[8 * c + 2 * i + 1] = h2f((uint16_t)(w[i] >> 16));
-            }
-        }
-    }
-}
-
-// Sum over aligned groups of L consecutive lanes (L a power of two <= 16):
-// every lane of the group gets the group's sum.
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-    if constexpr (L >= 2) v += dpp_f32<0xB1>(v);   // quad_perm [1,0,3,2]
-    if constexpr (L >= 4) v += dpp_f32<0x4E>(v);   // quad_perm [2,3,0,1]
-    if constexpr (L >= 8) v += __shfl_xor(v, 4, kWave);
-    if constexpr (L >= 16) v += __shfl_xor(v, 8, kWave);
-    return v;
-}
-
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// grid: (n_heads_kv * group / G, n_seq); block: waves * 64 (G > 1: 4 waves;
-// G == 1: up to 16).
-// LDS: waves * G * 64 floats (scores / probabilities), then the merge area
-// waves * G * (HD + 2) floats.
-template <typename TKV, int HD, int G>
-__global__ __launch_bounds__(G == 1 ? 1024 : 256) void attn_decode_kernel(
-    float* __restrict__ out, int64_t ld_out, const float* __restrict__ q, int64_t ld_q,
-    const TKV* __restrict__ kc, const TKV* __restrict__ vc, int64_t ld_pos, int64_t ld_seq,
-    const int32_t* __restrict__ lens, int n_past, int group, float scale) {
-    // lens[s] is clamped to [0, n_past] (n_past = the cache's positions)
-    // lanes per position: G * DPQ <= 64 q registers and a K slice of <= 32
-    constexpr int LPP = (HD * G / 64) > (HD / 32) ? (HD * G / 64) : (HD / 32);
-    constexpr int DPQ = HD / LPP;                                // q/k dims per lane
-    constexpr int PPP = kWave / LPP;                             // positions per pass
-    constexpr int NPASS = kAtTile / PPP;
-    constexpr int DPL = HD / kWave;                              // P V dims per lane
-    static_assert(LPP <= 16 && DPQ * G <= 64 && DPQ >= 8 && DPQ <= 32, "tile shape");
-    extern __shared__ float at_lds[];
-    const int waves = blockDim.x / kWave;
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int s = blockIdx.y;
-    const int h0 = blockIdx.x * G;      // first query head of this workgroup
-    const int j = h0 / group;           // its kv head
-    const int len = lens ? min(max(lens[s], 0), n_past) : n_past;
-    float* sc = at_lds + wave * G * kAtTile;  // this wave's scores [G][64]
-
-    const TKV* kb = kc + (int64_t)s * ld_seq + (int64_t)j * HD;
-    const TKV* vb = vc + (int64_t)s * ld_seq + (int64_t)j * HD;
-    const int sub = lane % LPP;  // which DPQ-slice of the row this lane holds
-
-    float qv[G][DPQ];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const float* qh = q + (int64_t)s * ld_q + (int64_t)(h0 + g) * HD + sub * DPQ;
-#pragma unroll
-        for (int c = 0; c < DPQ / 4; ++c) {
-            const float4 v = reinterpret_cast<const float4*>(qh)[c];
-            qv[g][4 * c] = v.x; qv[g][4 * c + 1] = v.y; qv[g][4 * c + 2] = v.z; qv[g][4 * c + 3] = v.w;
-        }
-    }
-
-    float m[G], l[G], acc[G][DPL];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m[g] = -INFINITY;
-        l[g] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) acc[g][i] = 0.0f;
-    }
-
-    for (int t0 = wave * kAtTile; t0 < len; t0 += waves * kAtTile) {
-        // scores of the tile
-#pragma unroll 2
-        for (int pass = 0; pass < NPASS; ++pass) {
-            const int pt = pass * PPP + lane / LPP;  // position within the tile
-            const int pos = t0 + pt < len ? t0 + pt : len - 1;
-            float kf[DPQ];
-            load_row<TKV, DPQ>(kb + (int64_t)pos * ld_pos + sub * DPQ, kf);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float d = 0.0f;
-#pragma unroll
-                for (int i = 0; i < DPQ; ++i) d = fmaf(qv[g][i], kf[i], d);
-                d = group_sum<LPP>(d);
-                if (sub == 0) sc[g * kAtTile + pt] = t0 + pt < len ? d * scale : -INFINITY;
-            }
-        }
-        wave_lds_sync();
-        // online softmax over the tile: lane = position
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const float st = sc[g * kAtTile + lane];
-            const float mn = fmaxf(m[g], wave_max_f32(st));  // finite: position t0 is live
-            const float corr = exp_neg_fast(m[g] - mn);             // 0 on the first tile
-            const float p = exp_neg_fast(st - mn);
-            l[g] = fmaf(l[g], corr, wave_sum_f32(p));
-            m[g] = mn;
-            sc[g * kAtTile + lane] = p;
-#pragma unroll
-            for (int i = 0; i < DPL; ++i) acc[g][i] *= corr;
-        }
-        wave_lds_sync();
-        // P V, 8 positions at a time with their V loads issued together
-        // (rows past the end re-read the last live row; their p is 0)
-        const int nt = len - t0 < kAtTile ? len - t0 : kAtTile;
-        const TKV* vt = vb + (int64_t)t0 * ld_pos + lane;
-        for (int t = 0; t < nt; t += 8) {
-            float vv[8][DPL];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int tt = t + u < nt ? t + u : nt - 1;
-#pragma unroll
-                for (int i = 0; i < DPL; ++i) vv[u][i] = KV<TKV>::get(vt + (int64_t)tt * ld_pos, i * kWave);
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const float p = sc[g * kAtTile + t + u];
-#pragma unroll
-                    for (int i = 0; i < DPL; ++i) acc[g][i] = fmaf(p, vv[u][i], acc[g][i]);
-                }
-        }
-        wave_lds_sync();
-    }
-
-    // merge the waves' states in wave order
-    float* mg = at_lds + waves * G * kAtTile;  // [waves][G][HD + 2]
-    constexpr int MS = HD + 2;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        float* e = mg + (wave * G + g) * MS;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) e[lane + i * kWave] = acc[g][i];
-        if (lane == 0) {
-            e[HD] = m[g];
-            e[HD + 1] = l[g];
-        }
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < G * HD; idx += blockDim.x) {
-        const int g = idx / HD, d = idx % HD;
-        float M = -INFINITY;
-        for (int w = 0; w < waves; ++w) M = fmaxf(M, mg[(w * G + g) * MS + HD]);
-        float num = 0.0f, den = 0.0f;
-        for (int w = 0; w < waves; ++w) {
-            const float* e = mg + (w * G + g) * MS;
-            const float f = exp_neg_fast(e[HD] - M);  // idle waves: m = -inf -> 0
-            num = fmaf(f, e[d], num);
-            den = fmaf(f, e[HD + 1], den);
-        }
-        out[(int64_t)s * ld_out + (int64_t)(h0 + g) * HD + d] = len > 0 ? num / den : 0.0f;
-    }
 }
 
 // Any head_dim (<= 1024) and alignment: one wave per (sequence, query head);
@@ -330,6 +142,7 @@ typedef float am_f4 __attribute__((ext_vector_type(4)));
 // sequences get short chunks; many sequences long ones).
 constexpr int kAmChunkMin = 256;
 constexpr int kAmTargetItems = 1024;
+constexpr int kF32Items = 128;         // fp32 caches: work items aimed for
 constexpr float kAmPScale = 32768.0f;  // 2^15
 // below this many (sequence, head group) pairs a split context is merged by
 // the attention kernel itself, at or above it by a second launch
@@ -344,85 +157,6 @@ __device__ __forceinline__ am_h8 am_h8_cat(am_h4 a, am_h4 b) {
 }
 
 __device__ __forceinline__ float ror8(float v) { return dpp_f32<0x128>(v); }  // row_ror:8
-
-// The in-kernel merge of a split context (attn_mfma_kernel with MERGE): the
-// calling workgroup has stored its records for head slots [h0, h0 + G) of
-// sequence s.  `lds` is the kernel's dynamic LDS, free at this point.
-template <int HD>
-__device__ __forceinline__ void am_merge_last(float* __restrict__ out, int64_t ld_out,
-                                              float* __restrict__ ws,
-                                              unsigned* __restrict__ counters, int s, int n_heads,
-                                              int h0, int G, int nch, int used, uint8_t* lds) {
-    constexpr int MS = HD + 2;
-    // The last of the `used` workgroups of this (sequence, head group) merges
-    // their records in chunk order and returns the counter to zero.  Records
-    // are written and read with device-coherent accesses (they bypass the
-    // per-XCD L2 caches, which are not coherent with one another).  Ordering:
-    // every thread waits for its record stores, the barrier (a workgroup-scope
-    // release / acquire) orders them before thread 0's counter update, an
-    // agent-scope release increment; the workgroup that sees the final count
-    // then acquires, so it synchronizes with every earlier release, and its
-    // threads read the records after the barrier that follows.  Only the
-    // merging workgroup pays the acquire's L2 invalidation.  (Agent-scope
-    // release fences in every wave instead cost 19 -> 28 us at batch 1, 8192
-    // positions: each writes back the whole L2.  A relaxed increment, relying
-    // on the device-coherent accesses alone, measured the same as this on the
-    // decode and 70B attention workloads.)
-    __shared__ int am_last;
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm<0>());
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned* cnt = counters + (int64_t)s * n_heads + blockIdx.x;
-        const unsigned prev =
-            __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        am_last = prev + 1 == (unsigned)used;
-        if (am_last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        if (am_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!am_last) return;
-    // Merge: the chunks' (m, l) pairs and weights f_c = exp(m_c - M) go
-    // through LDS (the tile buffers are free now), computed once per (chunk,
-    // head) in parallel; then each (head, dim) sums f_c O_c[d] over the chunks
-    // with the loads of several chunks in flight.  Same operations in the same
-    // order per output as a sequential merge.
-    float* mw = reinterpret_cast<float*>(lds);  // [used][8]: m, then f
-    float* ml = mw + used * 8;                  // [used][8]: l
-    float* mM = ml + used * 8;                  // [8]: M per head slot
-    for (int idx = threadIdx.x; idx < used * G; idx += blockDim.x) {
-        const int c = idx / G, g = idx % G;
-        const float* e = ws + (((int64_t)s * n_heads + h0 + g) * nch + c) * MS;
-        mw[c * 8 + g] = rec_load(e + HD);
-        ml[c * 8 + g] = rec_load(e + HD + 1);
-    }
-    __syncthreads();
-    if (threadIdx.x < G) {
-        float M = -INFINITY;
-        for (int c = 0; c < used; ++c) M = fmaxf(M, mw[c * 8 + threadIdx.x]);
-        mM[threadIdx.x] = M;
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < used * G; idx += blockDim.x) {
-        const int c = idx / G, g = idx % G;
-        const float M = mM[g];
-        mw[c * 8 + g] = M > -INFINITY ? exp_neg_fast(mw[c * 8 + g] - M) : 0.0f;
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < G * HD; idx += blockDim.x) {
-        const int g = idx / HD, d = idx % HD;
-        const float* rec = ws + ((int64_t)s * n_heads + h0 + g) * nch * MS + d;
-        float num = 0.0f, den = 0.0f;
-        if (mM[g] > -INFINITY) {
-#pragma unroll 8
-            for (int c = 0; c < used; ++c) {
-                const float f = mw[c * 8 + g];
-                num = fmaf(f, rec_load(rec + (int64_t)c * MS), num);
-                den = fmaf(f, ml[c * 8 + g], den);
-            }
-        }
-        out[(int64_t)s * ld_out + (int64_t)(h0 + g) * HD + d] = den > 0.0f ? num / den : 0.0f;
-    }
-}
 
 // grid (n_heads / G, n_seq, n_chunks), 256 threads.  ws == nullptr, or a
 // context that fits in one chunk: the workgroup writes the output directly;
@@ -868,12 +602,20 @@ __global__ __launch_bounds__(256) void am_clear_kernel(unsigned* __restrict__ c,
     if (i < n) c[i] = 0u;
 }
 
-template <int HD>
-static int am_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, const void* k,
-                     const void* v, int64_t ld_pos, int64_t ld_seq, const int32_t* lens,
-                     int n_past, int n_seq, int n_heads, int group, int G, float scale,
-                     const AmScratch& sc, MbXRec* xr, hipStream_t stream) {
-    const size_t shmem = (size_t)4 * 2 * kAtTile * HD * 2;  // K and V tile per wave
+// How a call splits its contexts: chunk positions per work item, and the
+// merge's counters and records (null when unsplit, or counters null when a
+// second launch merges).
+struct AmPlan {
+    bool split = false, in_kernel = false;
+    int chunk = 1, nch = 1, clear = 0;
+    unsigned* counters = nullptr;
+    float* ws = nullptr;
+};
+
+// lds: the kernel's LDS, which the in-kernel merge reuses.
+static AmPlan am_plan(const AmScratch& sc, int n_past, int n_seq, int n_heads, int G, int HD,
+                      size_t lds) {
+    AmPlan plan, *const p = &plan;
     // chunk: a multiple of 64 positions, at least kAmChunkMin, giving about
     // kAmTargetItems (sequence, head group, chunk) items
     const int64_t work = (int64_t)n_past * n_seq * (n_heads / G);
@@ -882,7 +624,7 @@ static int am_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, c
     if (ch < kAmChunkMin) ch = kAmChunkMin;
     // the merge keeps 16 floats per chunk (+ 8) in the tile buffers' LDS
     bool split = sc.base && n_past > ch &&
-                 ((n_past + ch - 1) / ch * 16 + 8) * sizeof(float) <= shmem;
+                 ((n_past + ch - 1) / ch * 16 + 8) * sizeof(float) <= lds;
     if (split && !sc.fixed && sc.bytes < am_workspace_bytes(n_seq, n_heads, HD, n_past))
         split = false;
     // The fixed scratch: a split whose records or in-launch merge counters do
@@ -897,31 +639,50 @@ static int am_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, c
             (ink && (size_t)n_seq * n_heads * sizeof(unsigned) > kScratchCounterBytes))
             split = false;
     }
-    const int chunk = split ? (int)ch : (n_past > 0 ? n_past : 1);
-    const int nch = split ? (n_past + chunk - 1) / chunk : 1;
+    p->split = split;
+    p->chunk = split ? (int)ch : (n_past > 0 ? n_past : 1);
+    p->nch = split ? (n_past + p->chunk - 1) / p->chunk : 1;
     // Few (sequence, head group) pairs: the last workgroup of each merges in
     // the same launch (measured at batch 1, 8192 positions: 19 us against 27
     // with a second launch).  Many: every chunk workgroup would wait on the
     // merge counter before retiring, so a separate wide merge launch is
     // faster (64 sequences x 8 groups: 268 us against 290).
     const bool in_kernel = (int64_t)n_seq * (n_heads / G) < kAmInKernelMerge;
-    unsigned* counters = nullptr;
-    float* ws = nullptr;
+    p->in_kernel = in_kernel;
     if (split && sc.fixed) {
         const size_t slots = (size_t)n_seq * n_heads;  // fits: checked above
-        counters = in_kernel ? static_cast<unsigned*>(sc.base) : nullptr;
-        ws = reinterpret_cast<float*>(static_cast<uint8_t*>(sc.base) + kScratchCounterBytes);
-        if (counters) {
-            // the scratch keeps the previous call's contents: clear the counters
-            const int st = launch(am_clear_kernel, dim3((unsigned)((slots + 255) / 256)),
-                                  dim3(256), 0, stream, counters, (int)slots);
-            if (st != JINF_HIP_OK) return st;
-        }
+        p->counters = in_kernel ? static_cast<unsigned*>(sc.base) : nullptr;
+        p->ws = reinterpret_cast<float*>(static_cast<uint8_t*>(sc.base) + kScratchCounterBytes);
+        p->clear = p->counters ? (int)slots : 0;
     } else if (split) {
-        counters = in_kernel ? static_cast<unsigned*>(sc.base) : nullptr;
-        ws = reinterpret_cast<float*>(static_cast<char*>(sc.base) +
+        p->counters = in_kernel ? static_cast<unsigned*>(sc.base) : nullptr;
+        p->ws = reinterpret_cast<float*>(static_cast<char*>(sc.base) +
                                       am_counter_bytes(n_seq, n_heads));
     }
+    return plan;
+}
+
+// The scratch keeps the previous call's contents: clear the counters the plan
+// uses.
+static int am_clear(const AmPlan& p, hipStream_t stream) {
+    if (p.clear <= 0) return JINF_HIP_OK;
+    return launch(am_clear_kernel, dim3((unsigned)((p.clear + 255) / 256)), dim3(256), 0, stream,
+                  p.counters, p.clear);
+}
+
+template <int HD>
+static int am_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, const void* k,
+                     const void* v, int64_t ld_pos, int64_t ld_seq, const int32_t* lens,
+                     int n_past, int n_seq, int n_heads, int group, int G, float scale,
+                     const AmScratch& sc, MbXRec* xr, hipStream_t stream) {
+    const size_t shmem = (size_t)4 * 2 * kAtTile * HD * 2;  // K and V tile per wave
+    const AmPlan p = am_plan(sc, n_past, n_seq, n_heads, G, HD, shmem);
+    const int pc = am_clear(p, stream);
+    if (pc != JINF_HIP_OK) return pc;
+    const bool split = p.split, in_kernel = p.in_kernel;
+    const int chunk = p.chunk, nch = p.nch;
+    unsigned* const counters = p.counters;
+    float* const ws = p.ws;
     // up to 128 positions per work item the four waves share each tile by
     // 16-row blocks (otherwise at most two waves would hold a tile)
     const bool rb = chunk <= 2 * kAtTile;
@@ -942,30 +703,6 @@ static int am_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, c
     if (st != JINF_HIP_OK || !split || in_kernel) return st;
     return launch(attn_combine_kernel, dim3(n_heads, n_seq), dim3(HD), 0, stream, out, ld_out,
                   (const float*)ws, lens, n_past, n_heads, HD, nch, chunk);
-}
-
-template <typename TKV, int HD, int G>
-static int at_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, const void* k,
-                     const void* v, int64_t ld_pos, int64_t ld_seq, const int32_t* lens,
-                     int n_past, int n_seq, int n_heads, int group, int waves, float scale,
-                     hipStream_t stream) {
-    const size_t shmem = ((size_t)waves * G * kAtTile + (size_t)waves * G * (HD + 2)) * 4;
-    return launch(attn_decode_kernel<TKV, HD, G>, dim3(n_heads / G, n_seq), dim3(waves * kWave),
-                  shmem, stream, out, ld_out, q, ld_q, static_cast<const TKV*>(k),
-                  static_cast<const TKV*>(v), ld_pos, ld_seq, lens, n_past, group, scale);
-}
-
-template <typename TKV, int HD>
-static int at_pick_g(int G, float* out, int64_t ld_out, const float* q, int64_t ld_q,
-                     const void* k, const void* v, int64_t ld_pos, int64_t ld_seq,
-                     const int32_t* lens, int n_past, int n_seq, int n_heads, int group,
-                     int waves, float scale, hipStream_t stream) {
-    switch (G) {
-        case 8: return at_launch<TKV, HD, 8>(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq, n_heads, group, waves, scale, stream);
-        case 4: return at_launch<TKV, HD, 4>(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq, n_heads, group, waves, scale, stream);
-        case 2: return at_launch<TKV, HD, 2>(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq, n_heads, group, waves, scale, stream);
-        default: return at_launch<TKV, HD, 1>(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq, n_heads, group, waves, scale, stream);
-    }
 }
 
 // Every sequence has n_past positions (the drop-in: lens == nullptr), or
@@ -1015,19 +752,28 @@ static int attention_decode(float* out, int64_t ld_out, const float* q, int64_t 
         return am_launch<128>(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq,
                               n_heads, group, G, scale, sc, xr, stream);
     }
-    // fp32 cache: enough (sequence, kv head) pairs: one workgroup per pair,
-    // all its query heads (up to 8) together.  Otherwise one query head per
-    // workgroup, with more waves when the (known) context is long.
-    int G = 1, waves = 4;  // G > 1 always runs 4 waves (its launch bound)
-    if ((int64_t)n_seq * n_heads_kv >= 128) {
-        G = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-    } else {
-        const int tiles = lens ? 64 : (n_past + kAtTile - 1) / kAtTile;
-        waves = tiles < 4 ? 4 : tiles > 16 ? 16 : tiles;
+    // fp32 cache: as many query heads of a group (up to 8) per workgroup as
+    // leave kF32Items work items (chunks included), or one; workgroups of one
+    // kv head then share its rows through L2 (1 sequence, 32 / 8 heads x 128:
+    // 256 positions in 8 items of 4 heads 9.6 us, 32 of one head 6.3; 4096
+    // positions in 128 items of 4 heads 14.2, 512 of one head 32).  The fixed
+    // scratch serves fp16 caches only: without a caller's workspace an fp32
+    // call runs unsplit, with the same bits through either entry point.
+    {
+        const AmScratch fsc = sc.fixed ? AmScratch{nullptr, 0, false} : sc;
+        AmPlan p;
+        int G = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+        for (;; G /= 2) {
+            p = am_plan(fsc, n_past, n_seq, n_heads, G, head_dim, 65536);
+            if (G == 1 || (int64_t)n_seq * (n_heads / G) * p.nch >= kF32Items) break;
+        }
+        const int st = attn_f32_launch(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past,
+                                       n_seq, head_dim, n_heads, group, G, p.chunk, p.nch, scale,
+                                       p.ws, p.counters, stream);
+        if (st != JINF_HIP_OK || !p.split || p.in_kernel) return st;
+        return launch(attn_combine_kernel, dim3(n_heads, n_seq), dim3(head_dim), 0, stream, out,
+                      ld_out, (const float*)p.ws, lens, n_past, n_heads, head_dim, p.nch, p.chunk);
     }
-    if (head_dim == 64)
-        return at_pick_g<float, 64>(G, out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq, n_heads, group, waves, scale, stream);
-    return at_pick_g<float, 128>(G, out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past, n_seq, n_heads, group, waves, scale, stream);
 }
 
 // 1/sqrt(head_dim) rounded once from fp64 (the reference uses rsqrtf).
