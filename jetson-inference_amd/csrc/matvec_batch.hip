@@ -41,10 +41,12 @@
 //
 // Split over the columns.  Small row counts give few workgroups, so the
 // slabs are split over k_splits workgroups per row group; each writes its
-// fp32 partial to the workspace with device-coherent stores and bumps the
-// group's counter, and the last one sums the partials in split order (the
-// result does not depend on which finished last), applies the epilogue and
-// resets the counter to zero.
+// fp32 partial to the workspace.  For residual adds and Q / K / V a later
+// launch sums the partials in split order and applies the epilogue.  For
+// plain stores and gate / up pairs the partials go out with device-coherent
+// stores, each workgroup bumps the group's counter, and the last one sums
+// them in split order (the result does not depend on which finished last),
+// applies the epilogue and resets the counter to zero.
 //
 // Epilogues (per output row r, token b): store; add into y (the residual
 // stream); SiLU(gate) * up for a gate / up pair; RoPE at the token's position
@@ -94,8 +96,8 @@ struct MbJob {
     int64_t ld_seq;
     float* part;           // split partials [n_groups][k_splits][2 * MT * 1024]
     uint32_t* counters;    // [n_groups]
-    float* dpart;          // kMbEpiAdd, deferred: partial sums [k_splits][n_batch][rows]
-    int64_t dstride;       // (split stride), merged by the next preparation
+    float* dpart;          // kMbEpiAdd / kMbEpiQKV, split columns: partial sums
+    int64_t dstride;       // [k_splits][n_batch][rows] and the split stride, merged later
     int x_ready;           // (host) x already prepared in xrec: no preparation launch
 };
 
@@ -303,7 +305,7 @@ __global__ __launch_bounds__(256) void mb_prepare_kernel(const float* __restrict
 // ---- merge of a deferred residual add ----
 //
 // h[b][c] += p_0[b][c] + p_1[b][c] + ... (split order, the order of the
-// GEMV's own merge) for the k partial arrays p_s = part + s * stride of a
+// GEMV's in-kernel merge) for the k partial arrays p_s = part + s * stride of a
 // deferred residual add ([n_batch][cols], cols a multiple of 256).  Grid
 // (slices of 2048 columns, n_batch), one lane per 8 columns, every
 // partial's load issued before the sums.  It also reduces each slice of the
@@ -432,7 +434,7 @@ struct MbQkvJobs {
 
 // The Q / K / V epilogue after deferred column splits: one lane per row pair
 // of one sequence of one job sums that job's k_splits partials in split order
-// (the order of the GEMV's own merge), then rotates and stores as above.
+// (the order of the in-kernel merge), then rotates and stores as above.
 __global__ __launch_bounds__(256) void mb_qkv_epilogue_kernel(MbQkvJobs js, RopeTheta th) {
     constexpr int SB = 8;  // partials loaded together
     int i = blockIdx.x * 256 + threadIdx.x;
@@ -862,10 +864,10 @@ __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_k
     auto local_of = [](int idx) { return (idx / (MT * 1024)) * 32 + (idx & 31); };
     if constexpr (EPI == kMbEpiAdd || EPI == kMbEpiQKV) {
         if (j.dpart) {
-            // deferred merge: this split's sums go to its own partial array,
+            // split columns: this split's sums go to its own partial array,
             // summed afterwards by a launch of its own (the residual add's
-            // merge ahead of the next preparation, the Q / K / V epilogue):
-            // no counter, no cross-workgroup merge here
+            // merge, alone or ahead of the next preparation; the Q / K / V
+            // epilogue): no counter, no cross-workgroup merge here
             float* dp = j.dpart + split * j.dstride;
 #pragma unroll
             for (int i = 0; i < PV; ++i) {
@@ -877,7 +879,7 @@ __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_k
             return;
         }
     }
-    if (j.k_splits > 1) {
+    if constexpr (EPI == kMbEpiStore || EPI == kMbEpiSwiGLU) if (j.k_splits > 1) {
         // partials in thread-contiguous order ([group][split][thread][PV]),
         // 16-byte device-coherent (sc1) stores and loads, all loads of the
         // merge issued together
@@ -977,6 +979,22 @@ __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_k
             mb_qkv_store(j, th, b, v0, pv[idx], pv[idx + 1]);
         }
     }
+}
+
+// y[b][r] += the split columns' partial sums, in split order: one lane per
+// output row of one sequence, grid (ceil(rows / 256), n_batch).
+__global__ __launch_bounds__(256) void mb_finish_add_kernel(float* __restrict__ y, int ld_y,
+                                                            int rows,
+                                                            const float* __restrict__ part, int k,
+                                                            int64_t stride) {
+    const int b = blockIdx.y, row = blockIdx.x * 256 + threadIdx.x;
+    if (row >= rows) return;
+    const float* p = part + (int64_t)b * rows + row;
+    float a = 0.0f;
+#pragma unroll 8
+    for (int s = 0; s < k; ++s) a += p[s * stride];
+    float* o = y + (int64_t)b * ld_y + row;
+    *o = *o + a;
 }
 
 // ---- host side ----
@@ -1138,7 +1156,7 @@ int mb_dispatch_t(MbJob& j, const MbShape& sh, const MbTheta<EPI>& th, const voi
 }
 
 template <int EPI>
-int mb_dispatch(int qtype, MbJob& j, const MbShape& sh, const MbTheta<EPI>& th,
+int mb_dispatch_q(int qtype, MbJob& j, const MbShape& sh, const MbTheta<EPI>& th,
                 const void* norm_w, int norm_f16, float eps, const MbDefer* pend,
                 hipStream_t stream) {
     switch (qtype) {
@@ -1147,6 +1165,38 @@ int mb_dispatch(int qtype, MbJob& j, const MbShape& sh, const MbTheta<EPI>& th,
         case kQ4_K: return mb_dispatch_t<kQ4_K, EPI>(j, sh, th, norm_w, norm_f16, eps, pend, stream);
         case kQ6_K: return mb_dispatch_t<kQ6_K, EPI>(j, sh, th, norm_w, norm_f16, eps, pend, stream);
         default: return JINF_HIP_ERR_INVALID;
+    }
+}
+
+// The launch.  Residual adds and Q / K / V projections with split columns
+// leave the splits' sums in the workspace's partials, finished by a launch of
+// their own: merged by each row group's last workgroup inside the GEMV, behind
+// agent-scope release / acquire counters, a layer's GEMVs took 101 against 87
+// us (Llama-3-8B widths, Q4_0, 32 sequences) and 132 against 112 (Q4_K_M, 7).
+// Plain stores and gate / up pairs, split only for small matrices, keep that
+// merge.
+template <int EPI>
+int mb_dispatch(int qtype, MbJob& j, const MbShape& sh, const MbTheta<EPI>& th,
+                const void* norm_w, int norm_f16, float eps, const MbDefer* pend,
+                hipStream_t stream) {
+    const bool finish = (EPI == kMbEpiAdd || EPI == kMbEpiQKV) && j.k_splits > 1 && !j.dpart;
+    if (finish) {
+        j.dpart = j.part;  // [k_splits][n_batch][rows]: no more than the merge's records
+        j.dstride = (int64_t)j.n_batch * j.rows;
+    }
+    const int rc = mb_dispatch_q<EPI>(qtype, j, sh, th, norm_w, norm_f16, eps, pend, stream);
+    if (rc != JINF_HIP_OK || !finish) return rc;
+    if constexpr (EPI == kMbEpiQKV) {
+        MbQkvJobs js{};
+        js.j[0] = j;
+        js.pairs[0] = j.n_batch * (j.rows / 2);
+        js.n = 1;
+        return launch(mb_qkv_epilogue_kernel, dim3((unsigned)((js.pairs[0] + 255) / 256)),
+                      dim3(256), 0, stream, js, th);
+    } else {
+        return launch(mb_finish_add_kernel, dim3((unsigned)((j.rows + 255) / 256), (unsigned)j.n_batch),
+                      dim3(256), 0, stream, j.y, j.ld_y, j.rows, static_cast<const float*>(j.part),
+                      j.k_splits, j.dstride);
     }
 }
 
@@ -1373,8 +1423,9 @@ static int qkv_rope_batch(const void* wq, const void* wk, const void* wv, int qt
         j.dpart = part;
         j.dstride = (int64_t)n_batch * rows;
     }
+    const bool own = j.dpart != nullptr;  // partials in the caller's part
     rc = mb_dispatch<kMbEpiQKV>(qtype, j, sh, th, norm_w, f16, eps, pend, stream);
-    if (rc != JINF_HIP_OK || !j.dpart) return rc;
+    if (rc != JINF_HIP_OK || !own) return rc;
     const int pairs = n_batch * (rows / 2);
     if (collect) {
         // finished by the caller's one epilogue launch for the layer

@@ -137,6 +137,29 @@ def test_matvec_batch_add(dev, qtype, n_batch):
     check(host(yd), want, 1e-5 * a + np.abs(want) * 2.0 ** -23, "y + W x")
 
 
+@pytest.mark.parametrize("rows,cols,n_batch", [(300, 2048, 1), (257, 4096, 7), (64, 14336, 64)])
+def test_matvec_batch_add_split_rows(dev, rows, cols, n_batch):
+    """Split columns summed by the finishing launch at the edges of its
+    256-row blocks, into rows of y with padding between them (left alone);
+    twice, in one workspace (the bar of test_matvec_batch_add for each add)."""
+    qtype = oracle.Q4_K
+    r = tu.rng(57 + rows + n_batch)
+    W = tu.quant_table(r, qtype, rows, cols)
+    X = tu.normal(r, (n_batch, cols), 0.0, 1.0, np.float32)
+    Y0 = tu.normal(r, (n_batch, rows + 8), 0.0, 4.0, np.float32)
+    ref, a = mv_rows(qtype, W, X)
+    yd, Wd, Xd = to_dev(Y0), to_dev(W), to_dev(X)
+    ws = jinf_amd.matvec_batch_workspace(rows, cols, n_batch)
+    want, bar = Y0[:, :rows], 0.0
+    for k in range(2):
+        say(f"matvec_batch_add split {rows}x{cols} batch {n_batch} pass {k}")
+        jinf_amd.matvec_batch_add(Wd, Xd, qtype, yd[:, :rows], workspace=ws)
+        want = (want + ref).astype(np.float32)
+        bar = bar + 1e-5 * a + np.abs(want) * 2.0 ** -23
+        check(host(yd)[:, :rows], want, bar, "y + W x")
+    assert tu.bits_equal(host(yd)[:, rows:], Y0[:, rows:])
+
+
 @pytest.mark.parametrize("qtype", QTYPES, ids=lambda q: NAMES[q])
 @pytest.mark.parametrize("g_dtype", [np.float32, np.float16], ids=["g32", "g16"])
 def test_rmsnorm_matvec_batch(dev, qtype, g_dtype):
