@@ -461,8 +461,7 @@ int create(jinf_hip_engine** out, const jinf_hip_engine_desc* desc, void* owned)
     e->kv_layer_bytes = (size_t)d.max_context * e->kv_dim * e->kv_es;
     e->arg_parts = (d.n_vocab + 4 * kArgThreads - 1) / (4 * kArgThreads);
     if (e->arg_parts > kArgMaxParts) e->arg_parts = kArgMaxParts;
-    if (d.kv_type == JINF_HIP_F16)
-        e->ws_bytes = jinf_attention_workspace_bytes(1, d.n_heads, e->head_dim, d.max_context);
+    e->ws_bytes = jinf_attention_workspace_bytes(1, d.n_heads, e->head_dim, d.max_context);
 
     // activation block layout
     size_t off = 0;
