@@ -41,12 +41,12 @@
 //
 // Split over the columns.  Small row counts give few workgroups, so the
 // slabs are split over k_splits workgroups per row group; each writes its
-// fp32 partial to the workspace.  For residual adds and Q / K / V a later
-// launch sums the partials in split order and applies the epilogue.  For
-// plain stores and gate / up pairs the partials go out with device-coherent
-// stores, each workgroup bumps the group's counter, and the last one sums
-// them in split order (the result does not depend on which finished last),
-// applies the epilogue and resets the counter to zero.
+// fp32 partial to the workspace.  For residual adds and Q / K / V of larger
+// matrices a later launch sums the partials in split order and applies the
+// epilogue.  Otherwise the partials go out with device-coherent stores, each
+// workgroup bumps the group's counter, and the last one sums them in split
+// order (the result does not depend on which finished last), applies the
+// epilogue and resets the counter to zero.
 //
 // Epilogues (per output row r, token b): store; add into y (the residual
 // stream); SiLU(gate) * up for a gate / up pair; RoPE at the token's position
@@ -528,7 +528,11 @@ __device__ __forceinline__ void mb_wait_w(int wave) {
 }
 
 template <int MT> constexpr int mb_occ() { return 2; }  // waves per SIMD the kernel is sized for
-template <int QT, int MT, int EPI, int NT, int WV, int KSW>
+// MERGE: split columns are merged in this launch.  An instantiation of its own
+// for residual adds and Q / K / V: the merge's code beside the partial stores,
+// even when not run, made the batch-32 step of the Q4_K_M layout 0.6% slower
+// (Q6_K down projection 27.3 -> 28.2 us).
+template <int QT, int MT, int EPI, int NT, int WV, int KSW, bool MERGE>
 __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_kernel(MbJob j, MbTheta<EPI> th) {
     constexpr int THREADS = 64 * WV;
     constexpr int ROWS = 32 * NT;
@@ -862,7 +866,7 @@ __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_k
         return mb_token(mt, r, ln >> 5);
     };
     auto local_of = [](int idx) { return (idx / (MT * 1024)) * 32 + (idx & 31); };
-    if constexpr (EPI == kMbEpiAdd || EPI == kMbEpiQKV) {
+    if constexpr (!MERGE) {
         if (j.dpart) {
             // split columns: this split's sums go to its own partial array,
             // summed afterwards by a launch of its own (the residual add's
@@ -879,7 +883,7 @@ __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_k
             return;
         }
     }
-    if constexpr (EPI == kMbEpiStore || EPI == kMbEpiSwiGLU) if (j.k_splits > 1) {
+    if constexpr (MERGE) if (j.k_splits > 1) {
         // partials in thread-contiguous order ([group][split][thread][PV]),
         // 16-byte device-coherent (sc1) stores and loads, all loads of the
         // merge issued together
@@ -1062,7 +1066,12 @@ size_t mb_ws_bytes(const MbShape& sh, int epi, int out_rows, int n_slabs, int mt
 template <int QT, int MT, int EPI, int NT, int WV, int KSW>
 int mb_launch_shape(MbJob& j, const MbTheta<EPI>& th, hipStream_t stream) {
     const dim3 grid((unsigned)(j.n_groups * j.k_splits));
-    return launch(matvec_batch_kernel<QT, MT, EPI, NT, WV, KSW>, grid, dim3(64 * WV),
+    if constexpr (EPI == kMbEpiAdd || EPI == kMbEpiQKV) {
+        if (j.dpart || j.k_splits == 1)
+            return launch(matvec_batch_kernel<QT, MT, EPI, NT, WV, KSW, false>, grid,
+                          dim3(64 * WV), mb_lds_bytes<QT, MT, NT, KSW>(), stream, j, th);
+    }
+    return launch(matvec_batch_kernel<QT, MT, EPI, NT, WV, KSW, true>, grid, dim3(64 * WV),
                   mb_lds_bytes<QT, MT, NT, KSW>(), stream, j, th);
 }
 
@@ -1173,13 +1182,22 @@ int mb_dispatch_q(int qtype, MbJob& j, const MbShape& sh, const MbTheta<EPI>& th
 // their own: merged by each row group's last workgroup inside the GEMV, behind
 // agent-scope release / acquire counters, a layer's GEMVs took 101 against 87
 // us (Llama-3-8B widths, Q4_0, 32 sequences) and 132 against 112 (Q4_K_M, 7).
-// Plain stores and gate / up pairs, split only for small matrices, keep that
+// Small launches, weights x splits below kMbMergeMax, keep the merge: there the
+// two launches are quicker on the GPU too (2048 x 2048 in 8 splits, Q4_0, 7
+// sequences, replayed from a graph: 9.5 against 12.5 us), but a caller that
+// issues such calls one by one waits for the host, which the extra launch
+// costs 2.5 us (13.8 against 12.6 us; 1024 x 1024 13.8 against 11.3).  Above,
+// the GPU is the longer of the two: 4096 x 2048 in 8 splits 13.8 against 15.4
+// us, 1024 x 4096 in 16 13.7 against 15.7, 2048 x 8192 13.7 against 19.5.
+// Plain stores and gate / up pairs, split only for small matrices, always
 // merge.
+constexpr int64_t kMbMergeMax = 3 << 24;
 template <int EPI>
 int mb_dispatch(int qtype, MbJob& j, const MbShape& sh, const MbTheta<EPI>& th,
                 const void* norm_w, int norm_f16, float eps, const MbDefer* pend,
                 hipStream_t stream) {
-    const bool finish = (EPI == kMbEpiAdd || EPI == kMbEpiQKV) && j.k_splits > 1 && !j.dpart;
+    const bool finish = (EPI == kMbEpiAdd || EPI == kMbEpiQKV) && j.k_splits > 1 && !j.dpart &&
+                        (int64_t)j.rows * j.n_slabs * kMbCols * j.k_splits >= kMbMergeMax;
     if (finish) {
         j.dpart = j.part;  // [k_splits][n_batch][rows]: no more than the merge's records
         j.dstride = (int64_t)j.n_batch * j.rows;

@@ -137,11 +137,12 @@ def test_matvec_batch_add(dev, qtype, n_batch):
     check(host(yd), want, 1e-5 * a + np.abs(want) * 2.0 ** -23, "y + W x")
 
 
-@pytest.mark.parametrize("rows,cols,n_batch", [(300, 2048, 1), (257, 4096, 7), (64, 14336, 64)])
+@pytest.mark.parametrize("rows,cols,n_batch", [(300, 4096, 1), (3071, 2048, 7), (3072, 2048, 7),
+                                               (1025, 4096, 7), (320, 14336, 64)])
 def test_matvec_batch_add_split_rows(dev, rows, cols, n_batch):
-    """Split columns summed by the finishing launch at the edges of its
-    256-row blocks, into rows of y with padding between them (left alone);
-    twice, in one workspace (the bar of test_matvec_batch_add for each add)."""
+    """Split columns merged by the GEMV (weights x splits below 3 * 2^24) or summed by
+    the finishing launch, at the edges of its 256-row blocks, into rows of y with
+    padding between them (left alone); twice, in one workspace (the bar of test_matvec_batch_add for each add)."""
     qtype = oracle.Q4_K
     r = tu.rng(57 + rows + n_batch)
     W = tu.quant_table(r, qtype, rows, cols)
