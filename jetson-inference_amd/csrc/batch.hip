@@ -728,7 +728,10 @@ extern "C" int jinf_hip_batch_prefill(jinf_hip_batch* b, int seq, const int32_t*
     // caller sees (of a borrowed cache only the last row's).
     if (n_tokens > b->n_seq && b->wide_state == 0) {
         b->wide_state = bat_wide_create(b) == JINF_HIP_OK ? 1 : -1;
-        if (b->wide_state < 0) bat_wide_release(b);
+        if (b->wide_state < 0) {
+            bat_wide_release(b);
+            (void)hipGetLastError();  // handled: prompts stay on the narrow path
+        }
     }
     const int step = b->wide_state == 1 ? b->pf.rows / b->n_seq * b->n_seq : 0;
     int32_t* rw = b->h_io + b->n_seq + 16;  // tokens, positions, lengths of a chunk
