@@ -238,7 +238,7 @@ def build_attention(torch, jinf, g, name, n_seq, max_ctx, nh, nkv, hd, lens, kv_
             sets.append(lambda q=q, k=k, v=v, lc=lc, o=o, ws=ws: jinf.attention_decode(
                 q, k, v, lc, nh, nkv, out=o, workspace=ws))
     return Kernel(name, nbytes, n_seq, "sequences", sets,
-                  "attn_mfma_kernel" if kv_dtype == torch.float16 else "attn_decode_kernel",
+                  "attn_mfma_kernel" if kv_dtype == torch.float16 else "attn_f32_kernel",
                   keep[-len(sets)][:4],
                   lambda o, q, k, v, lc: o.attention(q, k, v, lc, nh, nkv, hd))
 
@@ -1154,7 +1154,7 @@ _KERNEL_KEYS = [("ew_vec_kernel<unsigned short, 1", "swiglu"),
                 ("matvec_kernel<12, false, 0, 0,", "gemv_down"),
                 ("matvec_kernel<14, false, 0, 0,", "gemv_down"),
                 ("matvec_any_kernel", "gemv_generic"),
-                ("attn_decode_kernel", "gqa_attention"),
+                ("attn_f32_kernel", "gqa_attention"),
                 ("attn_mfma_kernel", "gqa_attention"),
                 ("attn_combine_kernel", "gqa_attention_combine"),
                 ("attn_decode_any_kernel", "gqa_attention_generic"),
