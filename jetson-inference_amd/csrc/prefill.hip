@@ -95,120 +95,143 @@ struct PfJob {
 
 // ---- x preparation ----
 
-// Per token: merges k pending partial sums into the row (written back), then
-// the row's RMSNorm factor (norm_w) and the power-of-two scale that puts its
-// largest prepared magnitude in [2^14, 2^15), as the batched GEMVs'
-// preparation does.
-__global__ __launch_bounds__(256) void pf_stats_kernel(float* __restrict__ x, int ld_x, int cols,
-                                                       const float* __restrict__ part, int k,
-                                                       int64_t stride,
-                                                       const void* __restrict__ norm_w,
-                                                       int norm_f16, float eps,
-                                                       float2* __restrict__ scale,
-                                                       float* __restrict__ inv_s) {
-    __shared__ double red[4];
-    __shared__ float redf[4];
-    const int t = blockIdx.x, tid = threadIdx.x;
-    float* xr = x + (int64_t)t * ld_x;
-    double ss = 0.0;
-    float m = 0.0f;
-    for (int g = tid; g < cols / 8; g += 256) {
-        float v[8], gw[8];
-        const float4 p = *reinterpret_cast<const float4*>(xr + 8 * g);
-        const float4 q = *reinterpret_cast<const float4*>(xr + 8 * g + 4);
-        v[0] = p.x; v[1] = p.y; v[2] = p.z; v[3] = p.w;
-        v[4] = q.x; v[5] = q.y; v[6] = q.z; v[7] = q.w;
-        mb_norm8(norm_w, norm_f16, g, gw);
-        if (k > 0) {
-            float sum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-            const float* pp = part + (int64_t)t * cols + 8 * g;
-            for (int s = 0; s < k; ++s) {
-                const float4 a = *reinterpret_cast<const float4*>(pp + s * stride);
-                const float4 b = *reinterpret_cast<const float4*>(pp + s * stride + 4);
-                sum[0] += a.x; sum[1] += a.y; sum[2] += a.z; sum[3] += a.w;
-                sum[4] += b.x; sum[5] += b.y; sum[6] += b.z; sum[7] += b.w;
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] += sum[e];
-            *reinterpret_cast<float4*>(xr + 8 * g) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4*>(xr + 8 * g + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            if (norm_w) ss = fma((double)v[e], (double)v[e], ss);
-            m = fmaxf(m, fabsf(v[e] * gw[e]));
-        }
+// Merges k pending partial sums into 8 columns of a row, in split order.
+__device__ __forceinline__ void pf_add_parts(float (&v)[8], const float* __restrict__ pp, int k,
+                                             int64_t stride) {
+    float sum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int s = 0; s < k; ++s) {
+        const float4 a = *reinterpret_cast<const float4*>(pp + s * stride);
+        const float4 b = *reinterpret_cast<const float4*>(pp + s * stride + 4);
+        sum[0] += a.x; sum[1] += a.y; sum[2] += a.z; sum[3] += a.w;
+        sum[4] += b.x; sum[5] += b.y; sum[6] += b.z; sum[7] += b.w;
     }
-    ss = wave_sum_f64(ss);
-    m = wave_max_f32(m);
-    if ((tid & (kWave - 1)) == 0) {
-        red[tid / kWave] = ss;
-        redf[tid / kWave] = m;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        ss = red[0];
-        m = redf[0];
 #pragma unroll
-        for (int i = 1; i < 4; ++i) {
-            ss += red[i];
-            m = fmaxf(m, redf[i]);
-        }
-        const float rs = norm_w ? rms_scale(ss, cols, eps) : 1.0f;
-        const int ex = mb_scale_exp(norm_w ? rs * m : m);
-        scale[t] = make_float2(rs, ldexpf(1.0f, 15 - ex));
-        inv_s[t] = ldexpf(1.0f, ex - 15);
-    }
+    for (int e = 0; e < 8; ++e) v[e] += sum[e];
 }
 
-// grid (slabs, 32-token tiles): one record.  Wave w converts k-steps 4 w ..
-// 4 w + 3; lane (token, half) its 8 columns of each, so every store is the
-// wave's whole 1 KiB fragment.
-__global__ __launch_bounds__(256) void pf_convert_kernel(const float* __restrict__ x, int ld_x,
-                                                         int T, int n_slabs,
+__device__ __forceinline__ void pf_load8(float (&v)[8], const float* p) {
+    const float4 a = *reinterpret_cast<const float4*>(p);
+    const float4 b = *reinterpret_cast<const float4*>(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void pf_store8(float* p, const float (&v)[8]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+
+// The pending merge alone: grid (ceil(cols / 2048), T).
+__global__ __launch_bounds__(256) void pf_merge_kernel(float* __restrict__ x, int ld_x, int cols,
+                                                       const float* __restrict__ part, int k,
+                                                       int64_t stride) {
+    const int t = blockIdx.y, g = blockIdx.x * 256 + threadIdx.x;
+    if (g >= cols / 8) return;
+    float* xr = x + (int64_t)t * ld_x + 8 * g;
+    float v[8];
+    pf_load8(v, xr);
+    pf_add_parts(v, part + (int64_t)t * cols + 8 * g, k, stride);
+    pf_store8(xr, v);
+}
+
+// One prompt token's whole preparation in one pass: the pending merge, the
+// row's RMSNorm factor (norm_w), the power-of-two scale that puts its largest
+// prepared magnitude in [2^14, 2^15), as the batched GEMVs' preparation does,
+// then its share of the records, from the row held in registers (NG groups of
+// 8 columns a thread).  What bounds it: with few tokens the chain load -
+// reduce - store and the launch, with many the bytes.  One launch for
+// statistics and one for the conversion (which read the row again) made the
+// 77-token prompt of 4 layers of 2048 / 8192 791 us, this one 719; 1000
+// tokens of 4096 / 14336 take the same either way (8.70 ms for 8 layers).  A
+// token owns 16 bytes of each 512-byte run of a record, so the 8 tokens of a
+// 128-byte line go to workgroups of one XCD, whose L2 joins them.  Tokens
+// past T, up to the next whole tile, are zeros.
+template <int NG>
+__global__ __launch_bounds__(256) void pf_prepare_kernel(float* __restrict__ x, int ld_x, int cols,
+                                                         int T, const float* __restrict__ part,
+                                                         int k, int64_t stride,
                                                          const void* __restrict__ norm_w,
-                                                         int norm_f16,
-                                                         const float2* __restrict__ scale,
+                                                         int norm_f16, float eps,
+                                                         float* __restrict__ inv_s,
                                                          uint8_t* __restrict__ rec) {
-    __shared__ float sums[8][33];
-    const int slab = blockIdx.x, mt = blockIdx.y;
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int tok = 32 * mt + (lane & 31), h = lane >> 5;
-    const bool live = tok < T;
-    const float2 sc = live ? scale[tok] : make_float2(1.0f, 1.0f);
-    uint8_t* r = rec + ((int64_t)mt * n_slabs + slab) * kPfRec;
-    const float* xr = x + (int64_t)(live ? tok : 0) * ld_x + slab * kMbCols + 8 * h;
-    float4 raw[4][2];
+    __shared__ double red[4];
+    __shared__ float redf[4];
+    __shared__ float2 fac;
+    const int xcd = blockIdx.x & 7, ix = blockIdx.x >> 3;
+    const int t = 8 * (8 * (ix >> 3) + xcd) + (ix & 7), tid = threadIdx.x;
+    const int ng = cols / 8;
+    const bool live = t < T;
+    float v[NG][8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = 4 * wave + i;
-        raw[i][0] = *reinterpret_cast<const float4*>(xr + 16 * t);
-        raw[i][1] = *reinterpret_cast<const float4*>(xr + 16 * t + 4);
+    for (int i = 0; i < NG; ++i) {
+        const int g = tid + 256 * i;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
+        if (live && g < ng) pf_load8(v[i], x + (int64_t)t * ld_x + 8 * g);
     }
-    float prev = 0.0f;
+    float2 sc = make_float2(1.0f, 1.0f);
+    if (live) {
+        double ss = 0.0;
+        float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = 4 * wave + i;
-        float v[8] = {raw[i][0].x, raw[i][0].y, raw[i][0].z, raw[i][0].w,
-                      raw[i][1].x, raw[i][1].y, raw[i][1].z, raw[i][1].w};
+        for (int i = 0; i < NG; ++i) {
+            const int g = tid + 256 * i;
+            if (g >= ng) break;
+            float gw[8];
+            mb_norm8(norm_w, norm_f16, g, gw);
+            if (k > 0) {
+                pf_add_parts(v[i], part + (int64_t)t * cols + 8 * g, k, stride);
+                pf_store8(x + (int64_t)t * ld_x + 8 * g, v[i]);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (norm_w) ss = fma((double)v[i][e], (double)v[i][e], ss);
+                m = fmaxf(m, fabsf(v[i][e] * gw[e]));
+            }
+        }
+        ss = wave_sum_f64(ss);
+        m = wave_max_f32(m);
+        if ((tid & (kWave - 1)) == 0) {
+            red[tid / kWave] = ss;
+            redf[tid / kWave] = m;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            ss = red[0];
+            m = redf[0];
+#pragma unroll
+            for (int i = 1; i < 4; ++i) {
+                ss += red[i];
+                m = fmaxf(m, redf[i]);
+            }
+            const float rs = norm_w ? rms_scale(ss, cols, eps) : 1.0f;
+            const int ex = mb_scale_exp(norm_w ? rs * m : m);
+            fac = make_float2(rs, ldexpf(1.0f, 15 - ex));
+            inv_s[t] = ldexpf(1.0f, ex - 15);
+        }
+        __syncthreads();
+        sc = fac;
+    }
+    // group g: slab g / 32, k-step (g % 32) / 2, half g & 1
+    uint8_t* rt = rec + (int64_t)(t >> 5) * (ng / 32) * kPfRec + 16 * (t & 31);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const int g = tid + 256 * i;
+        if (g >= ng) break;
         if (norm_w) {
 #pragma clang fp contract(off)
             float gw[8];
-            mb_norm8(norm_w, norm_f16, slab * (kMbCols / 8) + 2 * t + h, gw);
+            mb_norm8(norm_w, norm_f16, g, gw);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (v[e] * sc.x) * gw[e];
+            for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] * sc.x) * gw[e];
         }
-        if (!live) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-        }
-        // fragment slot (token lane & 31, half h) of k-step t, columns in the
-        // order (0, 4, 1, 5, 2, 6, 3, 7); the sums are of the split values
+        // columns in the order (0, 4, 1, 5, 2, 6, 3, 7); the sums are of the
+        // split values
         uint32_t hw[4], lw[4];
         float sum = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float a0 = v[e] * sc.y, a1 = v[4 + e] * sc.y;
+            const float a0 = v[i][e] * sc.y, a1 = v[i][4 + e] * sc.y;
             const _Float16 h0 = (_Float16)a0, h1 = (_Float16)a1;
             const _Float16 l0 = (_Float16)(a0 - (float)h0), l1 = (_Float16)(a1 - (float)h1);
             hw[e] = (uint32_t)__builtin_bit_cast(uint16_t, h0) |
@@ -217,31 +240,19 @@ __global__ __launch_bounds__(256) void pf_convert_kernel(const float* __restrict
                     ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
             sum += ((float)h0 + (float)l0) + ((float)h1 + (float)l1);
         }
-        uint8_t* fr = r + 2048 * t + 16 * lane;
+        uint8_t* r = rt + (int64_t)(g >> 5) * kPfRec;
+        uint8_t* fr = r + 1024 * (g & 30) + 512 * (g & 1);
         *reinterpret_cast<uint4*>(fr) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
         *reinterpret_cast<uint4*>(fr + 1024) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-        sum = xor32_sum(sum);
-        if (i & 1) {
-            if (h == 0) sums[t >> 1][lane & 31] = prev + sum;
+        // a 32-column sub-block is 4 consecutive lanes' groups
+        sum += dpp_f32<0xB1>(sum);  // the halves of a k-step
+        sum += dpp_f32<0x4E>(sum);  // its two k-steps
+        if ((g & 3) < 2) {
+            const float s = sum * kPfSumScale;
+            const _Float16 hi = (_Float16)s;
+            const _Float16 o = (g & 3) == 0 ? hi : (_Float16)(s - (float)hi);
+            *reinterpret_cast<_Float16*>(r + 32768 + 512 * (g & 1) + 2 * ((g & 31) >> 2)) = o;
         }
-        prev = sum;
-    }
-    __syncthreads();
-    if (wave == 0) {
-        uint32_t w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            _Float16 o[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float s = sums[2 * i + e][lane & 31] * kPfSumScale;
-                const _Float16 hi = (_Float16)s;
-                o[e] = h ? (_Float16)(s - (float)hi) : hi;
-            }
-            w[i] = (uint32_t)__builtin_bit_cast(uint16_t, o[0]) |
-                   ((uint32_t)__builtin_bit_cast(uint16_t, o[1]) << 16);
-        }
-        *reinterpret_cast<uint4*>(r + 32768 + 16 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
 
@@ -869,23 +880,27 @@ int pf_prepare(const PfBuf& b, float* x, int ld_x, int T, int cols, const void* 
                int norm_type, float eps, PfPend* pend, hipStream_t stream) {
     const int f16 = norm_w && norm_type == JINF_HIP_F16;
     const int k = pend ? pend->k : 0;
-    int rc = launch(pf_stats_kernel, dim3((unsigned)T), dim3(256), 0, stream, x, ld_x, cols,
-                    static_cast<const float*>(b.part), k, (int64_t)T * cols, norm_w, f16, eps,
-                    b.scale, b.inv_s);
-    if (rc != JINF_HIP_OK) return rc;
-    if (pend) pend->k = 0;
-    const int tiles = (T + kPfTile - 1) / kPfTile * (kPfTile / 32);
-    return launch(pf_convert_kernel, dim3((unsigned)(cols / kMbCols), (unsigned)tiles), dim3(256),
-                  0, stream, static_cast<const float*>(x), ld_x, T, cols / kMbCols, norm_w, f16,
-                  static_cast<const float2*>(b.scale), b.rec);
+    const unsigned tokens = (unsigned)((T + kPfTile - 1) / kPfTile * kPfTile);
+    const int ng = (cols / 8 + 255) / 256;
+    if (ng > 16) return JINF_HIP_ERR_INVALID;  // (the batch takes at most 32768 columns)
+    auto* kern = ng <= 1   ? pf_prepare_kernel<1>
+                 : ng <= 2 ? pf_prepare_kernel<2>
+                 : ng <= 4 ? pf_prepare_kernel<4>
+                 : ng <= 8 ? pf_prepare_kernel<8>
+                           : pf_prepare_kernel<16>;
+    const int rc = launch(kern, dim3(tokens), dim3(256), 0, stream, x, ld_x, cols, T,
+                          static_cast<const float*>(b.part), k, (int64_t)T * cols, norm_w, f16, eps,
+                          b.inv_s, b.rec);
+    if (rc == JINF_HIP_OK && pend) pend->k = 0;
+    return rc;
 }
 
 int pf_merge(const PfBuf& b, float* x, int ld_x, int T, int cols, PfPend* pend,
              hipStream_t stream) {
     if (pend->k == 0) return JINF_HIP_OK;
-    const int rc = launch(pf_stats_kernel, dim3((unsigned)T), dim3(256), 0, stream, x, ld_x, cols,
-                          static_cast<const float*>(b.part), pend->k, (int64_t)T * cols,
-                          nullptr, 0, 0.0f, b.scale, b.inv_s);
+    const int rc = launch(pf_merge_kernel, dim3((unsigned)((cols / 8 + 255) / 256), (unsigned)T),
+                          dim3(256), 0, stream, x, ld_x, cols, static_cast<const float*>(b.part),
+                          pend->k, (int64_t)T * cols);
     pend->k = 0;
     return rc;
 }

@@ -63,6 +63,24 @@ def test_engine_prefill(n, types, heads, kv):
         check(e.logits(), decode(ref, toks[n:]), kv, "after the prompt")
 
 
+# The x preparation holds a row in 1, 2, 4, 8 or 16 groups of 8 columns a
+# thread (2048 columns each): both sides of every step, with a norm (n_embd)
+# and without (n_ff), the last one the widest row taken.
+@pytest.mark.parametrize("n_embd,heads,n_ff", [
+    (256, (4, 2), 2048), (256, (4, 2), 2304), (256, (4, 2), 4352), (256, (4, 2), 8448),
+    (256, (4, 2), 16640), (256, (4, 2), 32768), (2304, (18, 2), 512), (4352, (34, 2), 512),
+])
+def test_row_widths(n_embd, heads, n_ff):
+    hp, W = mu.tiny_model(seed=n_ff + n_embd, n_layers=1, n_embd=n_embd, n_heads=heads[0],
+                          n_heads_kv=heads[1], n_ff=n_ff, n_vocab=301,
+                          types=dict.fromkeys(MATS, Q4_K))
+    toks = tokens(67, 301, n_ff)
+    ref = oeng.Decoder(hp, W, max_context=80, kv_type=F32)
+    with jinf_amd.Engine(hp, mu.to_device(W), 80, F32) as e:
+        e.prefill(toks)
+        check(e.logits(), decode(ref, toks), F32, f"{n_embd} / {n_ff}")
+
+
 def test_two_chunks_and_a_later_prompt():
     """A prompt of two wide chunks, then another at a position inside the
     context (an attention tile starting past its first row)."""
