@@ -282,8 +282,9 @@ int jinf_dequant_rows(void* out, int ld_out, const void* table, int qtype, int n
  * workgroups, which merge their partial results themselves; it
  * needs jinf_attention_workspace_bytes(n_seq, n_heads, head_dim, max_ctx)
  * bytes, zero-filled before its first use (every call leaves its merge
- * counters at zero again, so it is reused without clearing), and must not be
- * shared by calls running concurrently. */
+ * counters at zero again, so it is reused without clearing, by calls of any
+ * shapes it is large enough for), and must not be shared by calls running
+ * concurrently. */
 int jinf_attention_decode(float* out, int ld_out, const float* q, int ld_q,
                           const void* k_cache, const void* v_cache, int kv_type,
                           int64_t ld_pos, int64_t ld_seq, const int32_t* lens,
@@ -301,7 +302,7 @@ size_t jinf_attention_workspace_bytes(int n_seq, int n_heads, int head_dim, int 
  * arguments, results and kernels as jinf_attention_decode with a workspace
  * (bit-identical outputs); the split contexts keep their merge counters and
  * chunk records in a library-owned scratch array in device memory instead:
- * 16 KiB of counters plus 8 MiB of records, one copy per device, held until
+ * 256 bytes of counters plus 8 MiB of records, one copy per device, held until
  * the process ends.  Nothing is allocated or freed by the call.
  *   - The first call on a device looks the scratch up (hipGetSymbolAddress)
  *     with that device current; make each call with the stream's device

@@ -144,9 +144,6 @@ constexpr int kAmChunkMin = 256;
 constexpr int kAmTargetItems = 1024;
 constexpr int kF32Items = 128;         // fp32 caches: work items aimed for
 constexpr float kAmPScale = 32768.0f;  // 2^15
-// below this many (sequence, head group) pairs a split context is merged by
-// the attention kernel itself, at or above it by a second launch
-constexpr int kAmInKernelMerge = 128;
 
 __device__ __forceinline__ am_h4 am_h4_from(uint32_t lo, uint32_t hi) {
     const uint2 u = make_uint2(lo, hi);
@@ -162,8 +159,8 @@ __device__ __forceinline__ float ror8(float v) { return dpp_f32<0x128>(v); }  //
 // context that fits in one chunk: the workgroup writes the output directly;
 // otherwise each (sequence, head, chunk) writes an unnormalised partial
 // {O[HD], m, l} to ws, and either the last workgroup of the (sequence, head
-// group) to finish merges them (counters: one per (sequence, head group),
-// zero between calls) or, counters == nullptr, attn_combine_kernel does.
+// group) to finish merges them (counters: those of am_merge_last, zero
+// between calls) or, counters == nullptr, attn_combine_kernel does.
 typedef short am_tr4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) am_tr4 am_lds_tr4;
 // The parameters the prologue needs before the first K / V loads lead the
@@ -558,26 +555,26 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
     out[(int64_t)s * ld_out + (int64_t)h * hd + d] = den > 0.0f ? num / den : 0.0f;
 }
 
-// Workspace: one merge counter per (sequence, head group) -- n_seq * n_heads
-// slots cover any grouping -- padded to 256 bytes, then the chunk records
-// {O[HD], m, l} of every (sequence, head, chunk).
-static size_t am_counter_bytes(int n_seq, int n_heads) {
-    return ((size_t)n_seq * n_heads * sizeof(unsigned) + 255) / 256 * 256;
+// Workspace: the merge counters in its first kAmCounterBytes, and from
+// am_rec_offset on the chunk records {O[HD], m, l} of every (sequence, head,
+// chunk).
+static size_t am_rec_offset(int n_seq, int n_heads) {
+    const size_t o = ((size_t)n_seq * n_heads * sizeof(unsigned) + 255) / 256 * 256;
+    return o > kAmCounterBytes ? o : kAmCounterBytes;
 }
 
 static size_t am_workspace_bytes(int n_seq, int n_heads, int head_dim, int max_ctx) {
     const int64_t nch = ((int64_t)max_ctx + kAmChunkMin - 1) / kAmChunkMin;
-    return am_counter_bytes(n_seq, n_heads) +
+    return am_rec_offset(n_seq, n_heads) +
            (size_t)n_seq * n_heads * nch * (head_dim + 2) * sizeof(float);
 }
 
 // Where a split context keeps its merge counters and chunk records.
 //   fixed == false: the caller's workspace (`base`, `bytes`), laid out as
 //     above and used only when it holds am_workspace_bytes for the call;
-//   fixed == true: this device's copy of `scratch` (below), with a fixed
-//     layout: kScratchCounterBytes of merge counters, then
-//     kScratchRecordBytes of records.  A call whose split needs more runs
-//     unsplit.
+//   fixed == true: this device's copy of `scratch` (below): the counters,
+//     then kScratchRecordBytes of records.  A call whose split needs more
+//     runs unsplit.
 struct AmScratch {
     void* base;
     size_t bytes;
@@ -585,15 +582,14 @@ struct AmScratch {
 };
 
 // The no-allocation entry point's scratch (jinf_attention_decode_noalloc):
-// 4096 merge counters and 8 MiB of chunk records, enough for every split of
+// the merge counters and 8 MiB of chunk records, enough for every split of
 // up to about 1000 (sequence, head group) pairs at head_dim 128 (the 70B
 // 64-sequence decode needs 4.3 MB).  Each device that runs the library holds
 // its own copy until the process ends; host code only ever passes the
 // per-device address from hipGetSymbolAddress (scratch_base), never the
 // symbol itself.
-constexpr size_t kScratchCounterBytes = (size_t)16 << 10;
 constexpr size_t kScratchRecordBytes = (size_t)8 << 20;
-static __device__ __align__(256) uint8_t scratch[kScratchCounterBytes + kScratchRecordBytes];
+static __device__ __align__(256) uint8_t scratch[kAmCounterBytes + kScratchRecordBytes];
 
 // Zero n merge counters (a kernel rather than a memset node, so that the
 // call stays correct when a caller captures it in a graph).
@@ -627,17 +623,14 @@ static AmPlan am_plan(const AmScratch& sc, int n_past, int n_seq, int n_heads, i
                  ((n_past + ch - 1) / ch * 16 + 8) * sizeof(float) <= lds;
     if (split && !sc.fixed && sc.bytes < am_workspace_bytes(n_seq, n_heads, HD, n_past))
         split = false;
-    // The fixed scratch: a split whose records or in-launch merge counters do
-    // not fit runs unsplit, as a call with too small a workspace does (such a
-    // split has about as many (sequence, head group) pairs as work items to
-    // aim for, so the unsplit launch still fills the GPU).
+    // The fixed scratch: a split whose records do not fit runs unsplit, as a
+    // call with too small a workspace does (such a split has about as many
+    // (sequence, head group) pairs as work items to aim for, so the unsplit
+    // launch still fills the GPU).
     if (split && sc.fixed) {
         const size_t need = (size_t)n_seq * n_heads * ((n_past + ch - 1) / ch) * (HD + 2) *
                             sizeof(float);
-        const bool ink = (int64_t)n_seq * (n_heads / G) < kAmInKernelMerge;
-        if (need > kScratchRecordBytes ||
-            (ink && (size_t)n_seq * n_heads * sizeof(unsigned) > kScratchCounterBytes))
-            split = false;
+        if (need > kScratchRecordBytes) split = false;
     }
     p->split = split;
     p->chunk = split ? (int)ch : (n_past > 0 ? n_past : 1);
@@ -649,15 +642,11 @@ static AmPlan am_plan(const AmScratch& sc, int n_past, int n_seq, int n_heads, i
     // faster (64 sequences x 8 groups: 268 us against 290).
     const bool in_kernel = (int64_t)n_seq * (n_heads / G) < kAmInKernelMerge;
     p->in_kernel = in_kernel;
-    if (split && sc.fixed) {
-        const size_t slots = (size_t)n_seq * n_heads;  // fits: checked above
+    if (split) {
         p->counters = in_kernel ? static_cast<unsigned*>(sc.base) : nullptr;
-        p->ws = reinterpret_cast<float*>(static_cast<uint8_t*>(sc.base) + kScratchCounterBytes);
-        p->clear = p->counters ? (int)slots : 0;
-    } else if (split) {
-        p->counters = in_kernel ? static_cast<unsigned*>(sc.base) : nullptr;
-        p->ws = reinterpret_cast<float*>(static_cast<char*>(sc.base) +
-                                      am_counter_bytes(n_seq, n_heads));
+        const size_t rec = sc.fixed ? kAmCounterBytes : am_rec_offset(n_seq, n_heads);
+        p->ws = reinterpret_cast<float*>(static_cast<char*>(sc.base) + rec);
+        p->clear = sc.fixed && in_kernel ? (int)(kAmCounterBytes / sizeof(unsigned)) : 0;
     }
     return plan;
 }

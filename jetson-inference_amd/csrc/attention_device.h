@@ -8,6 +8,15 @@
 
 namespace jinf {
 
+// Below kAmInKernelMerge (sequence, head group) pairs a split context is
+// merged by the attention kernel itself, at or above it by a second launch.
+// The merge's counters, one per pair, are 16-bit counts, two to a word, in
+// the first kAmCounterBytes of the workspace whatever the call's shape, and
+// every call's records start at or past them.  So calls of any shapes share a
+// workspace: none writes records where another one keeps its counters.
+constexpr int kAmInKernelMerge = 128;
+constexpr size_t kAmCounterBytes = kAmInKernelMerge * sizeof(uint16_t);
+
 // The in-kernel merge of a split context (the kernels' MERGE form): the
 // calling workgroup has stored its records for head slots [h0, h0 + G) of
 // sequence s.  `lds` is the kernel's dynamic LDS, free at this point.
@@ -35,12 +44,16 @@ __device__ __forceinline__ void am_merge_last(float* __restrict__ out, int64_t l
     __builtin_amdgcn_s_waitcnt(waitcnt_vm<0>());
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned* cnt = counters + (int64_t)s * n_heads + blockIdx.x;
+        // (a count stays below 2048: the merge's LDS bounds the chunks)
+        const unsigned i = s * gridDim.x + blockIdx.x, shift = 16 * (i & 1);
+        unsigned* cnt = counters + (i >> 1);
         const unsigned prev =
-            __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        am_last = prev + 1 == (unsigned)used;
+            __hip_atomic_fetch_add(cnt, 1u << shift, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        am_last = ((prev >> shift) & 0xFFFFu) + 1 == (unsigned)used;
         if (am_last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        if (am_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (am_last)
+            __hip_atomic_fetch_sub(cnt, (unsigned)used << shift, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     if (!am_last) return;
