@@ -454,17 +454,16 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
         const int g = idx / HD, d = idx % HD;
         float M = -INFINITY;
         for (int w = 0; w < 4; ++w) M = fmaxf(M, mg[(w * 8 + g) * MS + HD]);
+        const float Ms = softmax_ref(M);
         float num = 0.0f, den = 0.0f;
-        if (M > -INFINITY) {
-            for (int w = 0; w < 4; ++w) {
-                const float* e = mg + (w * 8 + g) * MS;
-                const float f = exp_neg_fast(e[HD] - M);
-                num = fmaf(f, e[d], num);
-                den = fmaf(f, e[HD + 1], den);
-            }
+        for (int w = 0; w < 4; ++w) {
+            const float* e = mg + (w * 8 + g) * MS;
+            const float f = exp_neg_fast(e[HD] - Ms);
+            num = fmaf(f, e[d], num);
+            den = fmaf(f, e[HD + 1], den);
         }
         if (direct) {
-            const float o = den > 0.0f ? num / den : 0.0f;
+            const float o = len > 0 ? num / den : 0.0f;
             out[(int64_t)s * ld_out + (int64_t)(h0 + g) * HD + d] = o;
             if (xrec) {
                 ov[idx] = o;
@@ -543,16 +542,15 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
     const float* rec = ws + ((int64_t)s * n_heads + h) * nch * (hd + 2);
     float M = -INFINITY;
     for (int c = 0; c < used; ++c) M = fmaxf(M, rec[c * (hd + 2) + hd]);
+    const float Ms = softmax_ref(M);
     float num = 0.0f, den = 0.0f;
-    if (M > -INFINITY) {
-        for (int c = 0; c < used; ++c) {
-            const float* e = rec + c * (hd + 2);
-            const float f = exp_neg_fast(e[hd] - M);
-            num = fmaf(f, e[d], num);
-            den = fmaf(f, e[hd + 1], den);
-        }
+    for (int c = 0; c < used; ++c) {
+        const float* e = rec + c * (hd + 2);
+        const float f = exp_neg_fast(e[hd] - Ms);
+        num = fmaf(f, e[d], num);
+        den = fmaf(f, e[hd + 1], den);
     }
-    out[(int64_t)s * ld_out + (int64_t)h * hd + d] = den > 0.0f ? num / den : 0.0f;
+    out[(int64_t)s * ld_out + (int64_t)h * hd + d] = num / den;
 }
 
 // Workspace: the merge counters in its first kAmCounterBytes, and from

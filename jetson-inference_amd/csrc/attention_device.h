@@ -17,6 +17,12 @@ namespace jinf {
 constexpr int kAmInKernelMerge = 128;
 constexpr size_t kAmCounterBytes = kAmInKernelMerge * sizeof(uint16_t);
 
+// Reference point of a row's exponentials: its largest score, or 0 when it
+// has none above -inf (then exp(-inf - 0) = 0, not NaN).  Maxima skip NaN
+// scores, so a row with one keeps it in its probability sum and outputs,
+// which stay NaN through every merge whatever the row's maximum is.
+__device__ __forceinline__ float softmax_ref(float m) { return m > -INFINITY ? m : 0.0f; }
+
 // The in-kernel merge of a split context (the kernels' MERGE form): the
 // calling workgroup has stored its records for head slots [h0, h0 + G) of
 // sequence s.  `lds` is the kernel's dynamic LDS, free at this point.
@@ -64,7 +70,7 @@ __device__ __forceinline__ void am_merge_last(float* __restrict__ out, int64_t l
     // order per output as a sequential merge.
     float* mw = reinterpret_cast<float*>(lds);  // [used][8]: m, then f
     float* ml = mw + used * 8;                  // [used][8]: l
-    float* mM = ml + used * 8;                  // [8]: M per head slot
+    float* mM = ml + used * 8;                  // [8]: reference point per head slot
     for (int idx = threadIdx.x; idx < used * G; idx += blockDim.x) {
         const int c = idx / G, g = idx % G;
         const float* e = ws + (((int64_t)s * n_heads + h0 + g) * nch + c) * MS;
@@ -75,28 +81,25 @@ __device__ __forceinline__ void am_merge_last(float* __restrict__ out, int64_t l
     if (threadIdx.x < G) {
         float M = -INFINITY;
         for (int c = 0; c < used; ++c) M = fmaxf(M, mw[c * 8 + threadIdx.x]);
-        mM[threadIdx.x] = M;
+        mM[threadIdx.x] = softmax_ref(M);
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < used * G; idx += blockDim.x) {
         const int c = idx / G, g = idx % G;
-        const float M = mM[g];
-        mw[c * 8 + g] = M > -INFINITY ? exp_neg_fast(mw[c * 8 + g] - M) : 0.0f;
+        mw[c * 8 + g] = exp_neg_fast(mw[c * 8 + g] - mM[g]);
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < G * HD; idx += blockDim.x) {
         const int g = idx / HD, d = idx % HD;
         const float* rec = ws + ((int64_t)s * n_heads + h0 + g) * nch * MS + d;
         float num = 0.0f, den = 0.0f;
-        if (mM[g] > -INFINITY) {
 #pragma unroll 8
-            for (int c = 0; c < used; ++c) {
-                const float f = mw[c * 8 + g];
-                num = fmaf(f, rec_load(rec + (int64_t)c * MS), num);
-                den = fmaf(f, ml[c * 8 + g], den);
-            }
+        for (int c = 0; c < used; ++c) {
+            const float f = mw[c * 8 + g];
+            num = fmaf(f, rec_load(rec + (int64_t)c * MS), num);
+            den = fmaf(f, ml[c * 8 + g], den);
         }
-        out[(int64_t)s * ld_out + (int64_t)(h0 + g) * HD + d] = den > 0.0f ? num / den : 0.0f;
+        out[(int64_t)s * ld_out + (int64_t)(h0 + g) * HD + d] = num / den;
     }
 }
 

@@ -145,12 +145,13 @@ __global__ __launch_bounds__(64 * kFwWaves, 2) void attn_f32_kernel(
             float tm = pr[g][0];
 #pragma unroll
             for (int p = 1; p < NP; ++p) tm = fmaxf(tm, pr[g][p]);
-            const float mn = fmaxf(m[g], across_max<LPP>(tm));  // position t0 is live
-            const float corr = exp_neg_fast(m[g] - mn);
+            const float mn = fmaxf(m[g], across_max<LPP>(tm));
+            const float ms = softmax_ref(mn);
+            const float corr = exp_neg_fast(m[g] - ms);
             float ts = 0.0f;
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                pr[g][p] = exp_neg_fast(pr[g][p] - mn);
+                pr[g][p] = exp_neg_fast(pr[g][p] - ms);
                 ts += pr[g][p];
             }
             l[g] = fmaf(l[g], corr, across_sum<LPP>(ts));
@@ -210,15 +211,14 @@ __global__ __launch_bounds__(64 * kFwWaves, 2) void attn_f32_kernel(
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < kFwWaves; ++w) M = fmaxf(M, mg[(w * G + g) * MS + HD]);
+        const float Ms = softmax_ref(M);
         float num = 0.0f, den = 0.0f;
-        if (M > -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < kFwWaves; ++w) {
-                const float* e = mg + (w * G + g) * MS;
-                const float f = exp_neg_fast(e[HD] - M);  // idle waves: 0
-                num = fmaf(f, e[d], num);
-                den = fmaf(f, e[HD + 1], den);
-            }
+        for (int w = 0; w < kFwWaves; ++w) {
+            const float* e = mg + (w * G + g) * MS;
+            const float f = exp_neg_fast(e[HD] - Ms);  // idle waves: 0
+            num = fmaf(f, e[d], num);
+            den = fmaf(f, e[HD + 1], den);
         }
         if (direct) {
             out[(int64_t)s * ld_out + (int64_t)(h0 + g) * HD + d] = len > 0 ? num / den : 0.0f;
