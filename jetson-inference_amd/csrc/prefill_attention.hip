@@ -302,6 +302,7 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
         for (int r = 0; r < 4; ++r) {
             const int s = 4 * (lg & 1) + r;  // the slot of row r
             const float den = __shfl(l, s, kWave);
+            const bool empty = __shfl(lim[g], s, kWave) == 0;
             const bool nan = __shfl((int)poison[g], s, kWave);
             int tok, head;
             row_of(g, s, tok, head);
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
                 float* o = out + (int64_t)tok * ld_out + (int64_t)head * HD + col;
 #pragma unroll
                 for (int n = 0; n < NB; ++n)
-                    o[16 * n] = nan ? NAN : den > 0.0f ? O[g][n][r] * (1.0f / kPaPScale) / den : 0.0f;
+                    o[16 * n] = empty ? 0.0f : nan ? NAN : O[g][n][r] * (1.0f / kPaPScale) / den;
             }
         }
     }

@@ -146,3 +146,22 @@ def test_nonfinite_token_leaves_earlier_rows_alone():
                     check(got[i], want[first + i], F16, f"row {i}")
                 elif first + i == at:
                     assert np.all(np.isnan(got[i])), f"row {i}"
+
+
+def test_nonfinite_keys_with_finite_values():
+    """NaN weights in one kv head's K projection (V finite): every query head
+    of that group reads NaN scores, so every logit is NaN, as in a batched
+    step and in the oracle's loop."""
+    hp, W = mu.tiny_model(seed=12, n_vocab=301, types=dict.fromkeys(MATS, Q8_0))
+    hd = hp["n_embd"] // hp["n_heads"]
+    wk = W["blk.0.attn_k.weight"][0]
+    wk[hd + 3, 0:2] = np.frombuffer(np.float16(np.nan).tobytes(), np.uint8)
+    toks = tokens(40, 301, 12)
+    ref = oeng.Decoder(hp, W, max_context=64, kv_type=F16)
+    assert np.all(np.isnan(decode(ref, toks)))
+    for n_seq in (16, 40):  # wide; one batched step
+        with jinf_amd.Engine(hp, mu.to_device(W), 8, F16) as e, \
+                jinf_amd.Batch(e, n_seq, 64, F16) as b:
+            b.prefill(0, toks)
+            rows = (len(toks) - 1) % n_seq + 1
+            assert np.all(np.isnan(b.logits()[:rows])), n_seq
