@@ -553,6 +553,13 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
     out[(int64_t)s * ld_out + (int64_t)h * hd + d] = num / den;
 }
 
+int attn_combine_launch(float* out, int64_t ld_out, const float* ws, const int32_t* lens,
+                        int n_past, int n_seq, int n_heads, int head_dim, int nch, int chunk,
+                        hipStream_t stream) {
+    return launch(attn_combine_kernel, dim3(n_heads, n_seq), dim3(head_dim), 0, stream, out,
+                  ld_out, ws, lens, n_past, n_heads, head_dim, nch, chunk);
+}
+
 // Workspace: the merge counters in its first kAmCounterBytes, and from
 // am_rec_offset on the chunk records {O[HD], m, l} of every (sequence, head,
 // chunk).
@@ -570,13 +577,15 @@ static size_t am_workspace_bytes(int n_seq, int n_heads, int head_dim, int max_c
 // Where a split context keeps its merge counters and chunk records.
 //   fixed == false: the caller's workspace (`base`, `bytes`), laid out as
 //     above and used only when it holds am_workspace_bytes for the call;
-//   fixed == true: this device's copy of `scratch` (below): the counters,
-//     then kScratchRecordBytes of records.  A call whose split needs more
-//     runs unsplit.
+//   fixed == true: memory of any contents, the counters (cleared by the call)
+//     in its first kAmCounterBytes, then records.  A call whose split needs
+//     more runs unsplit.
+//   f32 == false: fp16 caches only.
 struct AmScratch {
     void* base;
     size_t bytes;
     bool fixed;
+    bool f32 = true;
 };
 
 // The no-allocation entry point's scratch (jinf_attention_decode_noalloc):
@@ -621,14 +630,14 @@ static AmPlan am_plan(const AmScratch& sc, int n_past, int n_seq, int n_heads, i
                  ((n_past + ch - 1) / ch * 16 + 8) * sizeof(float) <= lds;
     if (split && !sc.fixed && sc.bytes < am_workspace_bytes(n_seq, n_heads, HD, n_past))
         split = false;
-    // The fixed scratch: a split whose records do not fit runs unsplit, as a
+    // A fixed scratch: a split whose records do not fit runs unsplit, as a
     // call with too small a workspace does (such a split has about as many
     // (sequence, head group) pairs as work items to aim for, so the unsplit
     // launch still fills the GPU).
     if (split && sc.fixed) {
         const size_t need = (size_t)n_seq * n_heads * ((n_past + ch - 1) / ch) * (HD + 2) *
                             sizeof(float);
-        if (need > kScratchRecordBytes) split = false;
+        if (sc.bytes < kAmCounterBytes || need > sc.bytes - kAmCounterBytes) split = false;
     }
     p->split = split;
     p->chunk = split ? (int)ch : (n_past > 0 ? n_past : 1);
@@ -688,8 +697,8 @@ static int am_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, c
                           scale, out, ld_out, ws, counters, xrec, xr ? xr->mt : 1);
     if (xr) xr->wrote = st == JINF_HIP_OK && xrec != nullptr;
     if (st != JINF_HIP_OK || !split || in_kernel) return st;
-    return launch(attn_combine_kernel, dim3(n_heads, n_seq), dim3(HD), 0, stream, out, ld_out,
-                  (const float*)ws, lens, n_past, n_heads, HD, nch, chunk);
+    return attn_combine_launch(out, ld_out, ws, lens, n_past, n_seq, n_heads, HD, nch, chunk,
+                               stream);
 }
 
 // Every sequence has n_past positions (the drop-in: lens == nullptr), or
@@ -743,23 +752,25 @@ static int attention_decode(float* out, int64_t ld_out, const float* q, int64_t 
     // leave kF32Items work items (chunks included), or one; workgroups of one
     // kv head then share its rows through L2 (1 sequence, 32 / 8 heads x 128:
     // 256 positions in 8 items of 4 heads 9.6 us, 32 of one head 6.3; 4096
-    // positions in 128 items of 4 heads 14.2, 512 of one head 32).  The fixed
-    // scratch serves fp16 caches only: without a caller's workspace an fp32
-    // call runs unsplit, with the same bits through either entry point.
+    // positions in 128 items of 4 heads 14.2, 512 of one head 32).  The
+    // library's scratch serves fp16 caches only: without a caller's workspace an
+    // fp32 call runs unsplit, with the same bits through either entry point.
     {
-        const AmScratch fsc = sc.fixed ? AmScratch{nullptr, 0, false} : sc;
+        const AmScratch fsc = sc.f32 ? sc : AmScratch{nullptr, 0, false};
         AmPlan p;
         int G = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
         for (;; G /= 2) {
             p = am_plan(fsc, n_past, n_seq, n_heads, G, head_dim, 65536);
             if (G == 1 || (int64_t)n_seq * (n_heads / G) * p.nch >= kF32Items) break;
         }
+        const int pc = am_clear(p, stream);
+        if (pc != JINF_HIP_OK) return pc;
         const int st = attn_f32_launch(out, ld_out, q, ld_q, k, v, ld_pos, ld_seq, lens, n_past,
                                        n_seq, head_dim, n_heads, group, G, p.chunk, p.nch, scale,
                                        p.ws, p.counters, stream);
         if (st != JINF_HIP_OK || !p.split || p.in_kernel) return st;
-        return launch(attn_combine_kernel, dim3(n_heads, n_seq), dim3(head_dim), 0, stream, out,
-                      ld_out, (const float*)p.ws, lens, n_past, n_heads, head_dim, p.nch, p.chunk);
+        return attn_combine_launch(out, ld_out, p.ws, lens, n_past, n_seq, n_heads, head_dim,
+                                   p.nch, p.chunk, stream);
     }
 }
 
@@ -805,6 +816,15 @@ int attention_decode_xrec(float* out, int ld_out, const float* q, int ld_q, cons
     return attention_decode(out, ld_out, q, ld_q, k_cache, v_cache, kv_type, ld_pos, ld_seq, lens,
                             max_ctx, n_seq, head_dim, n_heads, n_heads_kv, scale,
                             AmScratch{workspace, workspace_bytes, false}, stream, xr);
+}
+
+int attention_rows(float* out, int ld_out, const float* q, int ld_q, const void* k, const void* v,
+                   int kv_type, int64_t ld_pos, const int32_t* lens, int n_rows, int n_ctx,
+                   int head_dim, int n_heads, int n_heads_kv, void* scratch, size_t scratch_bytes,
+                   hipStream_t stream) {
+    return attention_decode(out, ld_out, q, ld_q, k, v, kv_type, ld_pos, 0, lens, n_ctx, n_rows,
+                            head_dim, n_heads, n_heads_kv, inv_sqrt_hd(head_dim),
+                            AmScratch{scratch, scratch_bytes, true}, stream);
 }
 
 // This device's address of `scratch`: looked up with hipGetSymbolAddress on
@@ -853,7 +873,8 @@ extern "C" int jinf_attention_decode_noalloc(float* out, int ld_out, const float
     if (st != JINF_HIP_OK) return st;
     return jinf::attention_decode(out, ld_out, q, ld_q, k_cache, v_cache, kv_type, ld_pos, ld_seq,
                                   lens, max_ctx, n_seq, head_dim, n_heads, n_heads_kv, scale,
-                                  jinf::AmScratch{base, 0, true}, stream);
+                                  jinf::AmScratch{base, jinf::kAmCounterBytes + jinf::kScratchRecordBytes,
+                                                  true, false}, stream);
 }
 
 // Drop-in for cuda/attention_kernel.cu:100-115: one sequence, fp32 cache

@@ -103,6 +103,12 @@ __device__ __forceinline__ void am_merge_last(float* __restrict__ out, int64_t l
     }
 }
 
+// Merges the chunk records [sequence][head][nch] of every row whose context
+// does not fit in one chunk (attn_combine_kernel).
+int attn_combine_launch(float* out, int64_t ld_out, const float* ws, const int32_t* lens,
+                        int n_past, int n_seq, int n_heads, int head_dim, int nch, int chunk,
+                        hipStream_t stream);
+
 // The fp32-cache kernel (attention_f32.hip): G query heads of a kv head per
 // workgroup, chunks of `chunk` positions; counters null: split contexts are
 // left to attn_combine_kernel.

@@ -396,11 +396,12 @@ int bat_enqueue_wide(jinf_hip_batch* b, int T, int seq, int new_pos, int head_ro
         }
         bool done_attn = false;
         BAT_TRY(pf_attention(b->w_attn, qd, b->w_q, qd, kc, vc, b->kv_type, b->kv_dim, lens, T,
-                             b->bound, b->head_dim, d.n_heads, d.n_heads_kv, s, &done_attn));
+                             new_pos, b->head_dim, d.n_heads, d.n_heads_kv, b->pf.part,
+                             b->pf.part_bytes, s, &done_attn));
         if (!done_attn)
-            BAT_TRY(attention_decode_xrec(b->w_attn, qd, b->w_q, qd, kc, vc, b->kv_type, b->kv_dim,
-                                          0, lens, T, b->bound, b->head_dim, d.n_heads,
-                                          d.n_heads_kv, 0.0f, nullptr, 0, nullptr, s));
+            BAT_TRY(attention_rows(b->w_attn, qd, b->w_q, qd, kc, vc, b->kv_type, b->kv_dim, lens,
+                                   T, new_pos, b->head_dim, d.n_heads, d.n_heads_kv, b->pf.part,
+                                   b->pf.part_bytes, s));
         BAT_TRY(pf_prepare(b->pf, b->w_attn, qd, T, qd, nullptr, 0, 0.0f, nullptr, s));
         BAT_TRY(pf_matmul(b->pf, w.attn_output, w.attn_output_type, T, n, qd, b->w_hidden, n, true,
                           &pend, s));

@@ -94,6 +94,13 @@ int attention_decode_xrec(float* out, int ld_out, const float* q, int ld_q, cons
                           int n_heads_kv, float scale, void* workspace, size_t workspace_bytes,
                           MbXRec* xr, hipStream_t stream);
 
+// jinf_attention_decode of the rows of one cache (sequence stride 0), long
+// contexts split through a scratch of any contents.
+int attention_rows(float* out, int ld_out, const float* q, int ld_q, const void* k, const void* v,
+                   int kv_type, int64_t ld_pos, const int32_t* lens, int n_rows, int n_ctx,
+                   int head_dim, int n_heads, int n_heads_kv, void* scratch, size_t scratch_bytes,
+                   hipStream_t stream);
+
 // Partial sums of a deferred residual add y += W x: part[s][b][r] for split
 // s < k, sequence b < n_batch, row r < rows (stride elements between splits);
 // ss / mx: room for the merge's statistics of the new rows, per 2048-row

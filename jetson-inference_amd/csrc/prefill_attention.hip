@@ -16,9 +16,18 @@
 // groups of 8 rows x {hi, lo} columns).  No cross-wave merge is needed, and
 // the tiles are double-buffered: 64 KiB at head_dim 128, two workgroups per
 // CU.  Later tokens have longer contexts, so their workgroups start first.
+//
+// Few tokens far into a context give few workgroups with many tiles each (65
+// tokens at position 8000: 40 of 127).  Their contexts are split over the
+// grid's third dimension; each chunk leaves {O, m, l} records like the decode
+// kernel's, merged by its combine launch.  Prompts of 4 layers of 4096 /
+// 14336, at position 8000: 65 tokens 1919 -> 1125 us, 128 2011 -> 1249, 256
+// 2490 -> 1899, 1000 unchanged; 2 tokens 1810 -> 958.  (Twice the workgroups
+// aimed for: 1180, 1315, 1956; chunks of 128: 1120, 1258, 1897, 2 tokens 1001.)
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "attention_device.h"
 #include "jinf_device.h"
 #include "jinf_host.h"
 #include "jinf/kernels_ext.h"
@@ -36,19 +45,23 @@ typedef __attribute__((address_space(3))) pa_tr4 pa_lds_tr4;
 constexpr int kPaTile = 64;            // positions per tile
 constexpr int kPaRows = 64;            // (token, head) rows per workgroup
 constexpr float kPaPScale = 32768.0f;  // 2^15: probabilities in fp16's normal range
+constexpr int kPaTarget = 512;         // workgroups (two per CU) that splits aim for
+constexpr int kPaChunkMin = 256;       // positions per chunk, at least
 
 __device__ __forceinline__ pa_h8 pa_cat(pa_h4 a, pa_h4 b) {
     return pa_h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 }
 
-// grid (token tiles, n_heads / G), 256 threads; group = query heads per kv
-// head (a multiple of G).
-template <int HD>
+// grid (token tiles, n_heads / G, chunks), 256 threads; group = query heads
+// per kv head (a multiple of G).  SPLIT: chunks of `chunk` positions (a
+// multiple of the tile); a row whose context fits in one is written directly,
+// else its chunks' records go to ws[token][head][chunk].
+template <int HD, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
     const int32_t* __restrict__ lens, int T, int n_ctx, int G, int group,
     const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t ld_pos,
     const float* __restrict__ q, int64_t ld_q, float scale, float* __restrict__ out,
-    int64_t ld_out) {
+    int64_t ld_out, int chunk, int n_heads, float* __restrict__ ws) {
     constexpr int KS = HD / 16;       // 4-dim groups of q per lane
     constexpr int DPG = HD / 4;       // dims per lane group in the score product
     constexpr int KLD = DPG / 8;      // 32-deep k-steps of the score product
@@ -100,6 +113,11 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
     __shared__ unsigned bad_rows[2][2];
     if (tid < 4) bad_rows[tid >> 1][tid & 1] = 0u;
 
+    // the workgroup's positions: c0 .. c1
+    const int c0 = SPLIT ? (int)blockIdx.z * chunk : 0;
+    const int c1 = SPLIT ? min(wg_lim, c0 + chunk) : wg_lim;
+    if (SPLIT && c0 > 0 && c0 >= wg_lim) return;  // (before any barrier, workgroup-uniform)
+
     const uint32_t rowb = (uint32_t)ld_pos * 2;
     const int nrec = (int)((uint32_t)wg_lim * rowb);
     const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
@@ -126,7 +144,7 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
         for (int i = 0; i < LD; ++i)
             lds_load16_buf(vrs, voff[i], so, kb + kPaTile * PITCH + 1024 * (wave * LD + i));
     };
-    if (wg_lim > 0) load_tile(0, 0);
+    if (c0 < c1) load_tile(c0, 0);
 
     // q scale as fp16 hi / lo B fragments: the lane's 8 dims DPG lg + 8 u .. + 7
     pa_h8 qf[2][KLD];
@@ -162,12 +180,12 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
         for (int n = 0; n < NB; ++n) O[g][n] = pa_f4{0.f, 0.f, 0.f, 0.f};
 
     int buf = 0;
-    for (int t0 = 0; t0 < wg_lim; t0 += kPaTile, buf ^= 1) {
+    for (int t0 = c0; t0 < c1; t0 += kPaTile, buf ^= 1) {
         // this tile has landed for every wave, and every wave has finished
         // with the other buffer
         __builtin_amdgcn_s_waitcnt(waitcnt_vm<0>());
         __syncthreads();
-        if (t0 + kPaTile < wg_lim) load_tile(t0 + kPaTile, buf ^ 1);
+        if (t0 + kPaTile < c1) load_tile(t0 + kPaTile, buf ^ 1);
         // A tile in which some row's context ends holds later tokens' V rows.
         // Their probabilities are 0, but 0 times a non-finite value is not:
         // such values are cleared in LDS, and rows that do attend to one give
@@ -306,6 +324,25 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
             const bool nan = __shfl((int)poison[g], s, kWave);
             int tok, head;
             row_of(g, s, tok, head);
+            if constexpr (SPLIT) {
+                const int len = __shfl(lim[g], s, kWave);
+                const float mx = __shfl(m[g], s, kWave);
+                if (len > chunk) {  // (its later chunks that hold positions, and the first)
+                    if (lg < 2 && tok < T && c0 < len) {
+                        float* rec = ws + (((int64_t)tok * n_heads + head) * gridDim.z + blockIdx.z) *
+                                              (HD + 2);
+#pragma unroll
+                        for (int n = 0; n < NB; ++n)
+                            rec[16 * n + col] = nan ? NAN : O[g][n][r] * (1.0f / kPaPScale);
+                        if (col == 0) {
+                            rec[HD] = mx;
+                            rec[HD + 1] = den;
+                        }
+                    }
+                    continue;
+                }
+                if (c0 > 0) continue;
+            }
             if (lg < 2 && tok < T) {
                 float* o = out + (int64_t)tok * ld_out + (int64_t)head * HD + col;
 #pragma unroll
@@ -319,21 +356,36 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(
 template <int HD>
 int pa_launch(float* out, int64_t ld_out, const float* q, int64_t ld_q, const void* k,
               const void* v, int64_t ld_pos, const int32_t* lens, int T, int n_ctx, int n_heads,
-              int group, float scale, hipStream_t stream) {
+              int group, float scale, float* ws, size_t ws_bytes, hipStream_t stream) {
     const int G = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-    const int TQ = kPaRows / G;
-    return launch(pf_attention_kernel<HD>, dim3((unsigned)((T + TQ - 1) / TQ), (unsigned)(n_heads / G)),
-                  dim3(256), 2 * 2 * kPaTile * HD * 2, stream, lens, T, n_ctx, G, group,
-                  static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), ld_pos, q, ld_q,
-                  scale, out, ld_out);
+    const int TQ = kPaRows / G, tiles = (T + TQ - 1) / TQ;
+    // As many chunks as leave kPaTarget workgroups, of kPaChunkMin positions
+    // or more, and as their records fit in ws.
+    int64_t nch = kPaTarget / ((int64_t)tiles * (n_heads / G));
+    const int64_t fit = (int64_t)(ws_bytes / ((size_t)T * n_heads * (HD + 2) * sizeof(float)));
+    if (nch > fit) nch = fit;
+    if (nch > n_ctx / kPaChunkMin) nch = n_ctx / kPaChunkMin;
+    int chunk = n_ctx;
+    if (nch > 1) {
+        chunk = (int)((n_ctx + nch - 1) / nch + kPaTile - 1) / kPaTile * kPaTile;
+        nch = (n_ctx + chunk - 1) / chunk;
+    }
+    const bool split = nch > 1;
+    auto* kern = split ? pf_attention_kernel<HD, true> : pf_attention_kernel<HD, false>;
+    const int rc = launch(kern, dim3((unsigned)tiles, (unsigned)(n_heads / G), split ? (unsigned)nch : 1u),
+                          dim3(256), 2 * 2 * kPaTile * HD * 2, stream, lens, T, n_ctx, G, group,
+                          static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), ld_pos, q,
+                          ld_q, scale, out, ld_out, chunk, n_heads, ws);
+    if (rc != JINF_HIP_OK || !split) return rc;
+    return attn_combine_launch(out, ld_out, ws, lens, n_ctx, T, n_heads, HD, (int)nch, chunk, stream);
 }
 
 }  // namespace
 
 int pf_attention(float* out, int64_t ld_out, const float* q, int64_t ld_q, const void* k,
                  const void* v, int kv_type, int64_t ld_pos, const int32_t* lens, int T,
-                 int n_ctx, int head_dim, int n_heads, int n_heads_kv, hipStream_t stream,
-                 bool* launched) {
+                 int n_ctx, int head_dim, int n_heads, int n_heads_kv, float* ws, size_t ws_bytes,
+                 hipStream_t stream, bool* launched) {
     *launched = false;
     // buffer offsets are 32 bits, reads and q rows 16-byte aligned
     if (kv_type != JINF_HIP_F16 || (head_dim != 64 && head_dim != 128) || !aligned(k, 16) ||
@@ -344,9 +396,9 @@ int pf_attention(float* out, int64_t ld_out, const float* q, int64_t ld_q, const
     const int group = n_heads / n_heads_kv;
     const int rc = head_dim == 64
                        ? pa_launch<64>(out, ld_out, q, ld_q, k, v, ld_pos, lens, T, n_ctx, n_heads,
-                                       group, scale, stream)
+                                       group, scale, ws, ws_bytes, stream)
                        : pa_launch<128>(out, ld_out, q, ld_q, k, v, ld_pos, lens, T, n_ctx, n_heads,
-                                        group, scale, stream);
+                                        group, scale, ws, ws_bytes, stream);
     *launched = rc == JINF_HIP_OK;
     return rc;
 }

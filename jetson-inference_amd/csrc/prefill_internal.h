@@ -63,12 +63,12 @@ int pf_qkv(const PfBuf& b, const void* wq, const void* wk, const void* wv, int q
            hipStream_t stream);
 
 // Attention of T rows of one sequence over its cache (k, v: its position 0;
-// at most n_ctx positions), row t over positions below lens[t].  *launched
-// false (status 0, nothing enqueued): a cache type, head size or alignment
-// it does not take.
+// at most n_ctx positions), row t over positions below lens[t].  ws: scratch
+// for the records of split contexts, any contents.  *launched false (status
+// 0, nothing enqueued): a cache type, head size or alignment it does not take.
 int pf_attention(float* out, int64_t ld_out, const float* q, int64_t ld_q, const void* k,
                  const void* v, int kv_type, int64_t ld_pos, const int32_t* lens, int T,
-                 int n_ctx, int head_dim, int n_heads, int n_heads_kv, hipStream_t stream,
-                 bool* launched);
+                 int n_ctx, int head_dim, int n_heads, int n_heads_kv, float* ws, size_t ws_bytes,
+                 hipStream_t stream, bool* launched);
 
 }  // namespace jinf

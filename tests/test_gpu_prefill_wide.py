@@ -94,6 +94,29 @@ def test_two_chunks_and_a_later_prompt():
         check(e.logits(), decode(ref, toks[1100:]), F16, "150 more")
 
 
+@pytest.mark.parametrize("kv", [F16, F32], ids=["f16", "f32"])
+@pytest.mark.parametrize("n_embd,heads", [(256, (4, 2)), (256, (2, 1)), (768, (6, 2))])
+def test_prompts_deep_in_a_context(n_embd, heads, kv):
+    """Prompts whose contexts the attention splits: 600 tokens (short rows
+    written directly, long ones merged), then 65, 130 and 200 at its end, and
+    2 tokens in a batch of one sequence; one, two and three query heads per
+    kv head, head sizes 64 and 128."""
+    hp, W = mu.tiny_model(seed=n_embd + heads[1], n_layers=1, n_embd=n_embd, n_heads=heads[0],
+                          n_heads_kv=heads[1], n_vocab=301)
+    parts = (600, 65, 130, 200, 2)
+    toks = tokens(sum(parts), 301, heads[0])
+    ref = oeng.Decoder(hp, W, max_context=1024, kv_type=kv)
+    want = [ref.step(t) for t in toks]
+    with jinf_amd.Engine(hp, mu.to_device(W), 1024, kv) as e, jinf_amd.Batch(e, 1, 1024, kv) as b:
+        at = 0
+        for n in parts:
+            e.prefill(toks[at:at + n])
+            b.prefill(0, toks[at:at + n])
+            at += n
+            check(e.logits(), want[at - 1], kv, f"engine, {n} tokens")
+            check(b.logits()[0], want[at - 1], kv, f"batch, {n} tokens")
+
+
 @pytest.mark.parametrize("n_seq,n", [(1, 40), (3, 131), (50, 120)])
 def test_batch_prefill_logits_rows(n_seq, n):
     """The batch's rows after a wide prompt: the last chunk of n_seq tokens'
