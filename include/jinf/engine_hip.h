@@ -209,7 +209,8 @@ int  jinf_hip_batch_forward(jinf_hip_batch* b, const int32_t* tokens, const floa
  * m = (n_tokens - 1) mod n_seq + 1 tokens occupy rows 0 .. m - 1 of the
  * batch's logits; *logits (may be NULL) receives the device
  * pointer of that row.  Status 5 when the prompt does not fit the sequence's
- * context or an id is outside [0, n_vocab).  The reference feeds a prompt
+ * context or an id is outside [0, n_vocab); on any error the sequence stays
+ * at its position.  The reference feeds a prompt
  * one token at a time (src/engine.cpp:684-760); per token the arithmetic is
  * that loop's. */
 int  jinf_hip_batch_prefill(jinf_hip_batch* b, int seq, const int32_t* tokens, int n_tokens,

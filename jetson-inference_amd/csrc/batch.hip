@@ -761,9 +761,11 @@ extern "C" int jinf_hip_batch_prefill(jinf_hip_batch* b, int seq, const int32_t*
         const int sc = hip_rc(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
         if (rc != JINF_HIP_OK) return rc;
         if (sc != JINF_HIP_OK) return sc;
-        b->h_pos[seq] = p0 + c + m;
         c += m;
     }
+    // the last chunk has written the device's position: a prompt that fails
+    // before it leaves the sequence at p0, here as there
+    b->h_pos[seq] = p0 + n_tokens;
     if (logits) *logits = b->logits + (int64_t)last * d.n_vocab;
     return JINF_HIP_OK;
 }

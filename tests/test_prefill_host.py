@@ -1,0 +1,38 @@
+"""The prompt path's host side on the CPU: prefill_host_driver.cpp defines the
+HIP calls the library makes and lets chosen ones fail."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = "/opt/rocm"
+
+
+@pytest.fixture(scope="module")
+def seen(tmp_path_factory):
+    """{observation: [value of the wide path, of batched steps]}"""
+    exe = str(tmp_path_factory.mktemp("host") / "driver")
+    lib = os.path.join(ROOT, "jetson-inference_amd")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-rdynamic",
+                    "-I", os.path.join(ROOT, "include"), "-I", ROCM + "/include",
+                    os.path.join(ROOT, "tests", "prefill_host_driver.cpp"), "-o", exe,
+                    "-L", lib, "-l:libjinf_hip.so", "-L", ROCM + "/lib", "-lamdhip64",
+                    f"-Wl,-rpath,{lib}:{ROCM}/lib"], check=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout
+    got = {}
+    for line in out.splitlines():
+        k, v = line.split()
+        got.setdefault(k, []).append(int(v))
+    assert got["engine"] == [0] and got["batch"] == [0, 0] and got["first"] == [0, 0]
+    return got
+
+
+def test_failed_prompt_leaves_the_sequence_where_it_was(seen):
+    """The device position is written by a prompt's last chunk only, so a
+    prompt that fails before it leaves the host's position alone too, and the
+    next call goes on from there."""
+    assert all(v != 0 for v in seen["failed"])
+    assert seen["n_past"] == [5, 5]
+    assert seen["again"] == [0, 0] and seen["from"] == [5, 5]
+    assert seen["n_past_after"] == [8, 8]
