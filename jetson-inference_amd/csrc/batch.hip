@@ -321,7 +321,20 @@ void bat_wide_release(jinf_hip_batch* b) {
     b->wide = nullptr;
 }
 
-// The wide prompt path's buffers: up to kPfMaxRows tokens.
+// The calling thread's stream capture mode set to relaxed for a scope: an
+// allocation in it is allowed beside another thread's capture of the global
+// mode, and does not invalidate that capture.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool ok = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~RelaxedCapture() {
+        if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+// The wide prompt path's buffers: up to kPfMaxRows tokens.  Made inside a
+// prompt call, whatever other threads are capturing: a refusal for that
+// reason would leave the batch on batched steps for good.
 int bat_wide_create(jinf_hip_batch* b) {
     const jinf_hip_engine_desc& d = *b->d;
     const int R = std::min(kPfMaxRows, (b->max_ctx + kPfTile - 1) / kPfTile * kPfTile);
@@ -342,6 +355,7 @@ int bat_wide_create(jinf_hip_batch* b) {
     const size_t o_inv = take_b(rows * 4);
     const size_t o_cs = take_b(rows * (size_t)b->head_dim / 2 * 8);
     const size_t o_part = take_b(pf_part_bytes()), o_rows = take_b(3 * rows * 4);
+    const RelaxedCapture relaxed;
     BAT_TRY(hip_rc(hipMalloc((void**)&b->wide, off), "hipMalloc"));
     BAT_TRY(hip_rc(hipHostMalloc((void**)&b->h_wide, 3 * rows * 4, hipHostMallocDefault),
                    "hipHostMalloc"));

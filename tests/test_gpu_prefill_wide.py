@@ -6,8 +6,11 @@ Bars as for the engine's other paths, relative to the logit scale: 1e-4 with
 an fp32 cache (fp32 sums), 4e-4 with an fp16 cache (a cached value may round
 to its other fp16 neighbour).
 """
+import threading
+
 import numpy as np
 import pytest
+import torch
 
 import jinf_amd
 import model_util as mu
@@ -188,3 +191,34 @@ def test_nonfinite_keys_with_finite_values():
             b.prefill(0, toks)
             rows = (len(toks) - 1) % n_seq + 1
             assert np.all(np.isnan(b.logits()[:rows])), n_seq
+
+
+@pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
+def test_first_wide_prompt_beside_a_capture(mode):
+    """The first wide prompt (which allocates) in one thread while another
+    captures a graph: both succeed, and the graph replays.  (Beside a capture
+    of the global mode no prompt succeeds: the call waits for its stream.)"""
+    hp, W = mu.tiny_model(seed=13, n_vocab=301)
+    toks = np.asarray(tokens(100, 301, 13), np.int32)
+    ref = oeng.Decoder(hp, W, max_context=128, kv_type=F16)
+    want = decode(ref, [int(t) for t in toks])
+    with jinf_amd.Engine(hp, mu.to_device(W), 8, F16) as e, \
+            jinf_amd.Batch(e, 8, 128, F16) as b:
+        x = torch.arange(64, device="cuda", dtype=torch.float32)
+        y = torch.zeros_like(x)
+        torch.cuda.synchronize()
+        rc = []
+        prompt = threading.Thread(target=lambda: rc.append(
+            jinf_amd.lib().jinf_hip_batch_prefill(b._h, 0, toks.ctypes.data, toks.size, None)))
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, capture_error_mode=mode):
+            y.add_(x)
+            prompt.start()
+            prompt.join()
+            y.add_(1.0)
+        assert rc == [0]
+        for k in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, (k + 1) * (x + 1.0))
+        check(b.logits()[(toks.size - 1) % 8], want, F16, "prompt beside a capture")

@@ -36,3 +36,11 @@ def test_failed_prompt_leaves_the_sequence_where_it_was(seen):
     assert seen["n_past"] == [5, 5]
     assert seen["again"] == [0, 0] and seen["from"] == [5, 5]
     assert seen["n_past_after"] == [8, 8]
+
+
+def test_prompt_allocates_in_relaxed_capture_mode(seen):
+    """The first wide prompt allocates its buffers: in the thread's relaxed
+    capture mode, so that another thread's capture of the global mode neither
+    refuses nor loses by it, and the thread's own mode is kept."""
+    assert seen["allocs"][0] == 2 and seen["strict_allocs"] == [0, 0]
+    assert seen["mode_kept"] == [1, 1]
