@@ -352,7 +352,7 @@ int bat_wide_create(jinf_hip_batch* b) {
     const size_t o_attn = take_b(rows * b->q_dim * 4), o_ff = take_b(rows * nff * 4);
     const size_t o_up = take_b(split_ffn ? rows * nff * 4 : 0);
     const size_t o_rec = take_b(pf_rec_bytes(R, (int)std::max(n, nff)));
-    const size_t o_inv = take_b(rows * 4);
+    const size_t o_inv = take_b(rows * (std::max(n, nff) / 256) * 4);
     const size_t o_cs = take_b(rows * (size_t)b->head_dim / 2 * 8);
     const size_t o_part = take_b(pf_part_bytes()), o_rows = take_b(3 * rows * 4);
     const RelaxedCapture relaxed;

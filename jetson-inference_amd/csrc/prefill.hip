@@ -6,8 +6,9 @@
 //
 // Arithmetic: that of the batched GEMVs (matvec_batch.hip).  The weights'
 // integer codes are exact in fp16, x is split into fp16 hi + lo under a
-// power-of-two scale per token (about 22 significant bits), the products run
-// on v_mfma_f32_32x32x16_f16 and block scales multiply the fp32 block sums.
+// power-of-two scale per token and 256-column slab (about 22 significant bits
+// of every element down to 2^-18 of its slab's largest), the products run on
+// v_mfma_f32_32x32x16_f16 and block scales multiply the fp32 block sums.
 //
 // What bounds it: with hundreds of tokens the matrix cores and the vector
 // ALUs' issue.  One 32-column block of a 32 x 32 tile is 4 matrix-core
@@ -20,18 +21,26 @@
 // tile: a workgroup takes 128 tokens x 256 weight rows and decodes each
 // weight once, into fragments in LDS that the two token halves' waves share;
 // a wave takes 64 tokens x 64 rows (2 x 2 tiles of 32 x 32).  1000 tokens
-// (Q4_0): 4096 x 14336 235 us, 28672 x 4096 565 us (1.0 and 0.83 PFLOP/s of
-// matrix-core work; a dense 8192-cube fp16 library product reaches 1.2 on the
+// (Q4_0): 4096 x 14336 235 us, 28672 x 4096 565 us, 485 on a faster card (1.0
+// and 0.83 PFLOP/s of matrix-core work; a dense 8192-cube fp16 library product reaches 1.2 on the
 // same card, and all-zero operands run 20% faster, so part of the distance to
 // the 2.4 of the probe is the clock under load); as 16 batched steps of 64
 // tokens the same products take 296 and 860 us.
 //
 // Sums: MFMA chains of one block (hi products first: the lo ones added first
-// measured a 35% larger error), scaled into a first-level sum of kPfFlush
-// slabs, those into a second: with one running sum over a 4096-column row the
-// error against fp64 was 25% above the batched steps', with two levels it is
-// theirs (q4_0 2.56e-7 against 2.54e-7 over two layers and the head; Q4_K,
-// whose codes are centred here, 2.7e-7 against 4.3e-7).
+// measured a 35% larger error), scaled into a first-level sum of a slab (Q6_K,
+// with twice the blocks: half a slab), those times the slab's 1 / s into a
+// second.  Relative error of a layer's logits against fp64, batched steps ->
+// here (1024 to 4096 columns, 72 and 300 tokens): Q4_0 and Q8_0 1.6-2.0e-7 ->
+// 0.93-1.00 of it, Q6_K 1.6-2.1e-7 -> 0.87-0.99, Q4_K 3.7-4.2e-7 -> 0.45-0.47.
+// (First-level sums of two slabs under one scale per row: 1 to 2% faster
+// (Q6_K 5%), but Q6_K up to 1.07, Q4_0 1.02, and small columns of the output
+// and down projections' inputs beside ones 2^22 times larger three to four
+// times the error; the batched steps scale each column split by itself.)
+// Q4_K's minimum goes in through its codes' centre: coefficient and 32-column
+// sums of x as fp16 hi + lo (the batched steps': fp32), which the centred
+// codes' smaller terms more than make up for (medians with every minimum
+// zeroed, where centring gains nothing: 0.97-1.07).
 //
 // Data movement per stage (64 columns): x fragments (hi and lo) go to LDS
 // with direct-to-LDS loads; each lane loads one 32-column block of one weight
@@ -65,7 +74,6 @@ namespace {
 constexpr int kPfRec = 33 * 1024;
 constexpr float kPfSumScale = 0.03125f;
 constexpr int kPfTarget = 256;  // workgroups (one per CU) that column splits aim for
-constexpr int kPfFlush = 2;     // slabs per first-level sum
 
 enum PfEpi { kPfAdd = 0, kPfSwiGLU = 1, kPfQKV = 2 };
 
@@ -80,7 +88,8 @@ struct PfJob {
     int accum;
     int64_t row_bytes;
     const uint8_t* rec;
-    const float* inv_s;
+    const float* inv_s;    // [n_slabs][ld_inv]
+    int ld_inv;
     float* y;
     int ld_y;
     float* part;           // partial sums of split tiles: [k_splits][T][rows] when
@@ -135,14 +144,17 @@ __global__ __launch_bounds__(256) void pf_merge_kernel(float* __restrict__ x, in
 }
 
 // One prompt token's whole preparation in one pass: the pending merge, the
-// row's RMSNorm factor (norm_w), the power-of-two scale that puts its largest
-// prepared magnitude in [2^14, 2^15), as the batched GEMVs' preparation does,
-// then its share of the records, from the row held in registers (NG groups of
+// row's RMSNorm factor (norm_w), per 256-column slab the power-of-two scale
+// that puts the slab's largest prepared magnitude in [2^14, 2^15), then the
+// row's share of the records, from the row held in registers (NG groups of
 // 8 columns a thread).  What bounds it: with few tokens the chain load -
 // reduce - store and the launch, with many the bytes.  One launch for
 // statistics and one for the conversion (which read the row again) made the
 // 77-token prompt of 4 layers of 2048 / 8192 791 us, this one 719; 1000
-// tokens of 4096 / 14336 take the same either way (8.70 ms for 8 layers).  A
+// tokens of 4096 / 14336 take the same either way (8.70 ms for 8 layers).  With
+// a scale per slab, half a wave's maximum, a row without a norm needs no
+// barrier: 28.5 -> 27.6 us for 1000 tokens of 14336 columns, 17.7 -> 16.8 of
+// 4096.  A
 // token owns 16 bytes of each 512-byte run of a record, so the 8 tokens of a
 // 128-byte line go to workgroups of one XCD, whose L2 joins them.  Tokens
 // past T, up to the next whole tile, are zeros.
@@ -152,11 +164,9 @@ __global__ __launch_bounds__(256) void pf_prepare_kernel(float* __restrict__ x, 
                                                          int k, int64_t stride,
                                                          const void* __restrict__ norm_w,
                                                          int norm_f16, float eps,
-                                                         float* __restrict__ inv_s,
+                                                         float* __restrict__ inv_s, int ld_inv,
                                                          uint8_t* __restrict__ rec) {
     __shared__ double red[4];
-    __shared__ float redf[4];
-    __shared__ float2 fac;
     const int xcd = blockIdx.x & 7, ix = blockIdx.x >> 3;
     const int t = 8 * (8 * (ix >> 3) + xcd) + (ix & 7), tid = threadIdx.x;
     const int ng = cols / 8;
@@ -169,48 +179,28 @@ __global__ __launch_bounds__(256) void pf_prepare_kernel(float* __restrict__ x, 
         for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
         if (live && g < ng) pf_load8(v[i], x + (int64_t)t * ld_x + 8 * g);
     }
-    float2 sc = make_float2(1.0f, 1.0f);
+    float rs = 1.0f;
     if (live) {
-        double ss = 0.0;
-        float m = 0.0f;
+        if (k > 0) {
 #pragma unroll
-        for (int i = 0; i < NG; ++i) {
-            const int g = tid + 256 * i;
-            if (g >= ng) break;
-            float gw[8];
-            mb_norm8(norm_w, norm_f16, g, gw);
-            if (k > 0) {
+            for (int i = 0; i < NG; ++i) {
+                const int g = tid + 256 * i;
+                if (g >= ng) break;
                 pf_add_parts(v[i], part + (int64_t)t * cols + 8 * g, k, stride);
                 pf_store8(x + (int64_t)t * ld_x + 8 * g, v[i]);
             }
+        }
+        if (norm_w) {
+            double ss = 0.0;  // (groups past the row hold zeros)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (norm_w) ss = fma((double)v[i][e], (double)v[i][e], ss);
-                m = fmaxf(m, fabsf(v[i][e] * gw[e]));
-            }
-        }
-        ss = wave_sum_f64(ss);
-        m = wave_max_f32(m);
-        if ((tid & (kWave - 1)) == 0) {
-            red[tid / kWave] = ss;
-            redf[tid / kWave] = m;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            ss = red[0];
-            m = redf[0];
+            for (int i = 0; i < NG; ++i)
 #pragma unroll
-            for (int i = 1; i < 4; ++i) {
-                ss += red[i];
-                m = fmaxf(m, redf[i]);
-            }
-            const float rs = norm_w ? rms_scale(ss, cols, eps) : 1.0f;
-            const int ex = mb_scale_exp(norm_w ? rs * m : m);
-            fac = make_float2(rs, ldexpf(1.0f, 15 - ex));
-            inv_s[t] = ldexpf(1.0f, ex - 15);
+                for (int e = 0; e < 8; ++e) ss = fma((double)v[i][e], (double)v[i][e], ss);
+            ss = wave_sum_f64(ss);
+            if ((tid & (kWave - 1)) == 0) red[tid / kWave] = ss;
+            __syncthreads();
+            rs = rms_scale(((red[0] + red[1]) + red[2]) + red[3], cols, eps);
         }
-        __syncthreads();
-        sc = fac;
     }
     // group g: slab g / 32, k-step (g % 32) / 2, half g & 1
     uint8_t* rt = rec + (int64_t)(t >> 5) * (ng / 32) * kPfRec + 16 * (t & 31);
@@ -223,15 +213,27 @@ __global__ __launch_bounds__(256) void pf_prepare_kernel(float* __restrict__ x, 
             float gw[8];
             mb_norm8(norm_w, norm_f16, g, gw);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] * sc.x) * gw[e];
+            for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] * rs) * gw[e];
         }
+        // the slab's scale: its 32 groups are the lanes of half a wave
+        float m = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[i][e]));
+        m = fmaxf(m, dpp_f32<0xB1>(m));
+        m = fmaxf(m, dpp_f32<0x4E>(m));
+        m = fmaxf(m, __shfl_xor(m, 4, kWave));
+        m = fmaxf(m, dpp_f32<0x128>(m));  // row_ror:8
+        m = fmaxf(m, __shfl_xor(m, 16, kWave));
+        const int ex = mb_scale_exp(m);
+        const float sc = ldexpf(1.0f, 15 - ex);
+        if ((g & 31) == 0) inv_s[(int64_t)(g >> 5) * ld_inv + t] = ldexpf(1.0f, ex - 15);
         // columns in the order (0, 4, 1, 5, 2, 6, 3, 7); the sums are of the
         // split values
         uint32_t hw[4], lw[4];
         float sum = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float a0 = v[i][e] * sc.y, a1 = v[i][4 + e] * sc.y;
+            const float a0 = v[i][e] * sc, a1 = v[i][4 + e] * sc;
             const _Float16 h0 = (_Float16)a0, h1 = (_Float16)a1;
             const _Float16 l0 = (_Float16)(a0 - (float)h0), l1 = (_Float16)(a1 - (float)h1);
             hw[e] = (uint32_t)__builtin_bit_cast(uint16_t, h0) |
@@ -379,7 +381,8 @@ struct PfShape {
     static constexpr int DB = NSC * 64 * NW * 4;
     static constexpr int CB = QT == kQ4_K ? 64 * NW * 36 : 0;  // hi and lo coefficients, factor
     static constexpr int SB = QT == kQ4_K ? TILES * 1024 : 0;
-    static constexpr int LDS = 2 * (XB + WB + DB + CB + SB);
+    static constexpr int IB = 1024;  // a slab's 1 / s of the 128 tokens (twice)
+    static constexpr int LDS = 2 * (XB + WB + DB + CB + SB + IB);
     static_assert(32 * TILES == kPfTile && LDS <= 160 * 1024, "shape");
 };
 
@@ -419,6 +422,7 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
     uint8_t* const dbuf = wbuf + 2 * S::WB;
     uint8_t* const cbuf = dbuf + 2 * S::DB;
     uint8_t* const sbuf = cbuf + 2 * S::CB;
+    uint8_t* const ibuf = sbuf + 2 * S::SB;
 
     // ---- weights: lane (row, block of the stage) loads 32 columns' bytes,
     // one stage ahead of decoding them into fragments, which is one stage
@@ -476,7 +480,8 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
         *reinterpret_cast<mb_h8*>(wdst + b * S::WB + (o >> 1) * 1024 + (o & 1) * 512) =
             pf_decode8<QT>(raw, o, wg);
     };
-    // x fragments of stage st (and, Q4_K, its slab's sums in the first)
+    // x fragments of stage st (and, in its slab's first, the tokens' 1 / s
+    // and, Q4_K, the slab's sums)
     auto issue_x = [&](int st) {
         const int slab = st >> 2;
         uint8_t* dst = xbuf + (st & 1) * S::XB;
@@ -488,6 +493,10 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
                             (2 * KST * (st & 3) + r) * 1024,
                         16u * lane, dst + a * 1024);
         }
+        if ((st & 3) == 0 && wave == 7)
+            pf_lds_load(reinterpret_cast<const uint8_t*>(j.inv_s + (int64_t)slab * j.ld_inv +
+                                                         mtile * kPfTile),
+                        16u * (lane & 31), ibuf + (slab & 1) * S::IB);
         if constexpr (QT == kQ4_K) {
             if ((st & 3) == 0 && wave < TILES)
                 pf_lds_load(j.rec + ((int64_t)(mtile * TILES + wave) * j.n_slabs + slab) * kPfRec + 32768,
@@ -495,23 +504,36 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
         }
     };
 
-    // Two-level sums: acc takes kPfFlush slabs' blocks, then is added to sum
-    // (and cleared), so no value is rounded more than 8 kPfFlush + slabs /
-    // kPfFlush times on its way.
+    // Two-level sums: acc takes the blocks of kFlush stages, in units of x s,
+    // then is scaled by the slab's 1 / s, added to sum and cleared.  A value
+    // is rounded by at most 8 (Q4_0, Q8_0; Q6_K, of 16-column blocks) or 9
+    // (Q4_K) block FMAs of a first-level sum and by the row's 2 or 1 flushes
+    // per slab, besides the matrix-core chains' own roundings.
+    constexpr int kFlush = QT == kQ6_K ? 2 : 4;
     mb_f16 acc[2][MT], sum[2][MT];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[i][mt] = sum[i][mt] = mb_f16{};
-    auto flush = [&]() {
+    auto flush = [&](int slab) {
+        const float* iv = reinterpret_cast<const float*>(ibuf + (slab & 1) * S::IB) +
+                          32 * mw * MT + 4 * h;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 w = *reinterpret_cast<const float4*>(iv + 32 * mt + 8 * q);
+                const float f[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        sum[i][mt][4 * q + e] = fmaf(acc[i][mt][4 * q + e], f[e], sum[i][mt][4 * q + e]);
+            }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sum[i][mt][r] += acc[i][mt][r];
-                acc[i][mt] = mb_f16{};
-            }
+            for (int mt = 0; mt < MT; ++mt) acc[i][mt] = mb_f16{};
     };
     // Q4_K: the finished slab's coefficient times sum products
     auto corrections = [&](int slab) {
@@ -557,10 +579,6 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
         const int sn = st + 2 < st1 ? st + 2 : st1 - 1;
         const PfRaw<QT> next = pf_load_raw<QT>(wrow, 2 * sn + wblk);
         const int nb = (st & 1) ^ 1;
-        if ((st & 3) == 0 && st > st0) {
-            corrections((st >> 2) - 1);
-            if (((st >> 2) - s0) % kPfFlush == 0) flush();
-        }
 
         const uint8_t* xs = xbuf + (st & 1) * S::XB + mw * MT * KST * 2048 + lane * 16;
         const uint8_t* ws = wbuf + (st & 1) * S::WB + 2 * n * KST * 1024 + lane * 16;
@@ -627,22 +645,16 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
             scale_tile(2 * MT - 1);
         }
         raw = next;
+        // (here, not after the barrier: the waves have drifted apart, and one
+        // wave's flush runs beside another's matrix-core work)
+        if ((st + 1) % kFlush == 0) {
+            if ((st & 3) == 3) corrections(st >> 2);
+            flush(st >> 2);
+        }
     }
-    corrections(s1 - 1);
-    flush();
 
-    // the finished sums, scaled by 1 / s
     const int tok0 = (mtile * TILES + mw * MT) * 32 + 4 * h;
     auto tok = [&](int mi, int r) { return tok0 + 32 * mi + 8 * (r >> 2) + (r & 3); };
-    mb_f16 fin[MT][2];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float inv = j.inv_s[tok(mt, r)];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) fin[mt][i][r] = sum[i][mt][r] * inv;
-        }
     if (!whole && !j.pend) {
         // a split tile's partial sums, finished by pf_finish_kernel
         float* p = j.part + ((int64_t)(tile - j.tail0) * j.k_splits + split) * (kPfTile * 256) +
@@ -653,7 +665,7 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    p[(32 * mi + 8 * (r >> 2) + (r & 3)) * 256 + 32 * i] = fin[mi][i][r];
+                    p[(32 * mi + 8 * (r >> 2) + (r & 3)) * 256 + 32 * i] = sum[i][mi][r];
         return;
     }
     if constexpr (EPI == kPfSwiGLU) {
@@ -665,7 +677,7 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
             for (int r = 0; r < 16; ++r)
                 if (tok(mi, r) < j.T)
                     j.y[(int64_t)tok(mi, r) * j.ld_y + row] =
-                        swiglu_exact(fin[mi][0][r], fin[mi][1][r]);
+                        swiglu_exact(sum[0][mi][r], sum[1][mi][r]);
     } else if constexpr (EPI == kPfAdd) {
         float* const y = whole ? j.y : j.part + (int64_t)split * j.T * j.rows;
         const int64_t ld = whole ? j.ld_y : j.rows;
@@ -680,7 +692,7 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
                 for (int r = 0; r < 16; ++r)
                     if (tok(mi, r) < j.T) {
                         float* p = y + (int64_t)tok(mi, r) * ld + row;
-                        *p = accum ? *p + fin[mi][i][r] : fin[mi][i][r];
+                        *p = accum ? *p + sum[i][mi][r] : sum[i][mi][r];
                     }
             }
     } else {
@@ -699,7 +711,7 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
             for (int mi = 0; mi < MT; ++mi)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const float own = fin[mi][i][r], other = dpp_f32<0xB1>(own);
+                    const float own = sum[i][mi][r], other = dpp_f32<0xB1>(own);
                     const int t = tok(mi, r);
                     if (t < j.T && row < j.rows) {
                         float v = own;
@@ -854,6 +866,7 @@ int pf_job(PfJob& j, const PfBuf& b, int qtype, int T, int rows, int cols, float
     j.row_bytes = (int64_t)(cols / e) * bytes;
     j.rec = b.rec;
     j.inv_s = b.inv_s;
+    j.ld_inv = b.rows;
     j.y = y;
     j.ld_y = ld_y;
     j.part = b.part;
@@ -890,7 +903,7 @@ int pf_prepare(const PfBuf& b, float* x, int ld_x, int T, int cols, const void* 
                            : pf_prepare_kernel<16>;
     const int rc = launch(kern, dim3(tokens), dim3(256), 0, stream, x, ld_x, cols, T,
                           static_cast<const float*>(b.part), k, (int64_t)T * cols, norm_w, f16, eps,
-                          b.inv_s, b.rec);
+                          b.inv_s, b.rows, b.rec);
     if (rc == JINF_HIP_OK && pend) pend->k = 0;
     return rc;
 }

@@ -193,6 +193,32 @@ def test_nonfinite_keys_with_finite_values():
             assert np.all(np.isnan(b.logits()[:rows])), n_seq
 
 
+@pytest.mark.parametrize("qt", [Q4_0, Q8_0], ids=["q4_0", "q8_0"])
+def test_small_columns_beside_large_ones(qt):
+    """One 256-column slab of the down projection's input 2^26 times the rest,
+    against zero weights: the other columns keep their 22 bits (each slab is
+    split under a scale of its own).  Bar 2^-18 of the logit scale, four bits
+    for the sums; under one scale per row the columns keep 14 bits."""
+    hp, W = mu.tiny_model(seed=14, n_layers=1, n_embd=256, n_ff=2048, n_vocab=301,
+                          types=dict.fromkeys(MATS, qt))
+    bs = {Q4_0: 18, Q8_0: 34}[qt]
+    up = W["blk.0.ffn_up.weight"][0].reshape(2048, 256 // 32, bs)
+    d = np.ascontiguousarray(up[:256, :, :2]).view(np.float16).astype(np.float32)
+    up[:256, :, :2] = (d * 2.0 ** 26 / 2.0 ** 10).astype(np.float16).view(np.uint8)
+    gate = W["blk.0.ffn_gate.weight"][0].reshape(2048, 256 // 32, bs)
+    d = np.ascontiguousarray(gate[:256, :, :2]).view(np.float16).astype(np.float32)
+    gate[:256, :, :2] = (d * 2.0 ** 10).astype(np.float16).view(np.uint8)
+    W["blk.0.ffn_down.weight"][0].reshape(256, 2048 // 32, bs)[:, :8, :2] = 0
+    toks = tokens(72, 301, 14)
+    ref = oeng.Decoder(hp, W, max_context=80, kv_type=F32)
+    want = decode(ref, toks)
+    with jinf_amd.Engine(hp, mu.to_device(W), 80, F32) as e:
+        e.prefill(toks)
+        err = float(np.max(np.abs(e.logits().astype(np.float64) - want)))
+    print(f"error / scale {err / np.max(np.abs(want)):.2e}", flush=True)
+    assert err <= 2.0 ** -18 * float(np.max(np.abs(want)))
+
+
 @pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
 def test_first_wide_prompt_beside_a_capture(mode):
     """The first wide prompt (which allocates) in one thread while another
