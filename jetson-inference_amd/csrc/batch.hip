@@ -444,6 +444,28 @@ int bat_enqueue_wide(jinf_hip_batch* b, int T, int seq, int new_pos, int head_ro
     return bat_prefill_end(b, head_rows, seq, new_pos);
 }
 
+// Whether a prompt of more than one step is quicker as two batched steps than
+// as a wide one.  A wide step costs a layer about the same for 2 tokens as for
+// 64, so from three steps on it is always the quicker (1.2 times and more);
+// against two the weights' bytes decide: both read them, a batched step is
+// bound by it in large layers, a wide one by the decode.  A layer's time, wide
+// over two steps of up to 32 rows (Q4_0 / Q4_K_M / Q8_0):
+//    60M weights (2048 / 8192)    0.79-0.89 / 0.85-0.92 / 0.78-0.92
+//   113M (3072 / 8192)            0.70-0.82 / 0.74-0.85 / 0.71-0.78
+//   202M (4096 / 11008, 32 kv heads) 0.91-1.00 / 0.91-0.99 / 0.85-0.95
+//   218M (4096 / 14336)           1.01-1.05 / 0.98-1.03 / 0.94-0.99
+//   855M (8192 / 28672)           1.03-1.09 / 0.94-0.98
+// and over two steps of 64 rows 0.65-0.90 everywhere.  So two steps for large
+// layers of Q4_0, the format with the fewest bytes per weight decoded.
+constexpr int64_t kTwoStepWeights = 25 << 23;  // 210M
+bool bat_two_steps(const jinf_hip_batch* b, int n_tokens) {
+    const jinf_hip_engine_desc& d = *b->d;
+    const int64_t weights =
+        (int64_t)d.n_embd * (2 * b->q_dim + 2 * b->kv_dim + 3 * (int64_t)d.n_ff);
+    return n_tokens <= 2 * b->n_seq && b->n_seq <= 32 && weights >= kTwoStepWeights &&
+           d.n_layers > 0 && d.layers[0].ffn_gate_type == kQ4_0;
+}
+
 int bat_enqueue_step(jinf_hip_batch* b) { return bat_enqueue_rows(b, b->n_seq, -1, 0); }
 
 int bat_capture(jinf_hip_batch* b, hipGraphExec_t* out) {
@@ -737,17 +759,18 @@ extern "C" int jinf_hip_batch_prefill(jinf_hip_batch* b, int seq, const int32_t*
                  n_tokens, seq, p0, b->max_ctx);
         return JINF_HIP_ERR_INVALID;
     }
-    // Prompts longer than one batched step run wide: chunks of a multiple of
-    // n_seq tokens, so that the last chunk holds the rows whose logits the
-    // caller sees (of a borrowed cache only the last row's).
-    if (n_tokens > b->n_seq && b->wide_state == 0) {
+    // Prompts longer than one batched step (two, see below) run wide: chunks of
+    // a multiple of n_seq tokens, so that the last chunk holds the rows whose
+    // logits the caller sees (of a borrowed cache only the last row's).
+    const bool go_wide = n_tokens > b->n_seq && !bat_two_steps(b, n_tokens);
+    if (go_wide && b->wide_state == 0) {
         b->wide_state = bat_wide_create(b) == JINF_HIP_OK ? 1 : -1;
         if (b->wide_state < 0) {
             bat_wide_release(b);
             (void)hipGetLastError();  // handled: prompts stay on the narrow path
         }
     }
-    const int step = b->wide_state == 1 ? b->pf.rows / b->n_seq * b->n_seq : 0;
+    const int step = go_wide && b->wide_state == 1 ? b->pf.rows / b->n_seq * b->n_seq : 0;
     int32_t* rw = b->h_io + b->n_seq + 16;  // tokens, positions, lengths of a chunk
     int last = 0;
     for (int c = 0; c < n_tokens;) {

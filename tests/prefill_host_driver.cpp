@@ -116,5 +116,27 @@ int main() {
         jinf_hip_batch_destroy(b);
     }
     jinf_hip_engine_destroy(e);
+
+    // which prompts run wide: those whose first call allocates
+    const int widths[3][5] = {
+        {256, 512, 4, 2, 2}, {4096, 14336, 32, 8, 2}, {4096, 14336, 32, 8, 8}};  // 8: Q8_0
+    for (const auto& wd : widths) {
+        d.n_embd = wd[0];
+        d.n_ff = wd[1];
+        d.n_heads = wd[2];
+        d.n_heads_kv = wd[3];
+        lw.ffn_gate_type = lw.ffn_up_type = wd[4];
+        show("engine", jinf_hip_engine_create(&e, &d));
+        const int calls[5][2] = {{8, 8}, {8, 9}, {8, 16}, {8, 17}, {64, 65}};
+        for (const auto& c : calls) {
+            jinf_hip_batch* b = nullptr;
+            show("batch", jinf_hip_batch_create(&b, e, c[0], 256, 1));
+            g_allocs = 0;
+            show("first", jinf_hip_batch_prefill(b, 0, toks.data(), c[1], nullptr));
+            show("wide", g_allocs != 0);
+            jinf_hip_batch_destroy(b);
+        }
+        jinf_hip_engine_destroy(e);
+    }
     return 0;
 }

@@ -24,7 +24,7 @@ def seen(tmp_path_factory):
     for line in out.splitlines():
         k, v = line.split()
         got.setdefault(k, []).append(int(v))
-    assert got["engine"] == [0] and got["batch"] == [0, 0] and got["first"] == [0, 0]
+    assert not any(got["engine"] + got["batch"] + got["first"])
     return got
 
 
@@ -44,3 +44,10 @@ def test_prompt_allocates_in_relaxed_capture_mode(seen):
     refuses nor loses by it, and the thread's own mode is kept."""
     assert seen["allocs"][0] == 2 and seen["strict_allocs"] == [0, 0]
     assert seen["mode_kept"] == [1, 1]
+
+
+def test_which_prompts_run_wide(seen):
+    """8, 9, 16 and 17 tokens at 8 sequences and 65 at 64: more than one
+    batched step runs wide, with large Q4_0 layers more than two steps of up
+    to 32 rows."""
+    assert seen["wide"] == [0, 1, 1, 1, 1] + [0, 0, 0, 1, 1] + [0, 1, 1, 1, 1]
