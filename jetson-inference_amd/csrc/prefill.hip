@@ -806,7 +806,7 @@ __global__ __launch_bounds__(256) void pf_finish_kernel(PfJob j) {
 // tiles all fit in one round leaves its splits' sums pending instead, merged
 // by the next preparation's pass over the residual stream.
 template <int QT, int EPI>
-int pf_launch(PfJob& j, hipStream_t stream) {
+int pf_launch(PfJob& j, size_t part_bytes, hipStream_t stream) {
     using S = PfShape<QT>;
     constexpr int NW = S::NW;
     const int per_tile = EPI == kPfSwiGLU ? 32 * NW : 64 * NW;
@@ -823,6 +823,9 @@ int pf_launch(PfJob& j, hipStream_t stream) {
     j.full_per_xcd = j.tail0 / 8;
     j.tail_items = tail * j.k_splits;
     j.tail_per_xcd = (j.tail_items + 7) / 8;
+    const size_t tile_rows = j.pend ? (size_t)j.T * j.rows : (size_t)tail * kPfTile * 256;
+    if (j.k_splits > 1 && j.k_splits * tile_rows * sizeof(float) > part_bytes)
+        return JINF_HIP_ERR_INVALID;  // (the buffer holds kPfTarget split tiles)
     const int rc = launch(pf_matmul_kernel<QT, EPI>, dim3(8 * (j.full_per_xcd + j.tail_per_xcd)),
                           dim3(512), S::LDS, stream, j);
     if (rc != JINF_HIP_OK || j.k_splits == 1 || tail == 0 || j.pend) return rc;
@@ -830,12 +833,12 @@ int pf_launch(PfJob& j, hipStream_t stream) {
 }
 
 template <int EPI>
-int pf_dispatch(int qtype, PfJob& j, hipStream_t stream) {
+int pf_dispatch(int qtype, PfJob& j, const PfBuf& b, hipStream_t stream) {
     switch (qtype) {
-        case kQ4_0: return pf_launch<kQ4_0, EPI>(j, stream);
-        case kQ8_0: return pf_launch<kQ8_0, EPI>(j, stream);
-        case kQ4_K: return pf_launch<kQ4_K, EPI>(j, stream);
-        case kQ6_K: return pf_launch<kQ6_K, EPI>(j, stream);
+        case kQ4_0: return pf_launch<kQ4_0, EPI>(j, b.part_bytes, stream);
+        case kQ8_0: return pf_launch<kQ8_0, EPI>(j, b.part_bytes, stream);
+        case kQ4_K: return pf_launch<kQ4_K, EPI>(j, b.part_bytes, stream);
+        case kQ6_K: return pf_launch<kQ6_K, EPI>(j, b.part_bytes, stream);
         default: return JINF_HIP_ERR_INVALID;
     }
 }
@@ -925,7 +928,7 @@ int pf_matmul(const PfBuf& b, const void* w, int qtype, int T, int rows, int col
     if (rc != JINF_HIP_OK) return rc;
     j.accum = accum;
     j.pend = accum && pend;
-    rc = pf_dispatch<kPfAdd>(qtype, j, stream);
+    rc = pf_dispatch<kPfAdd>(qtype, j, b, stream);
     if (pend) pend->k = rc == JINF_HIP_OK && j.pend ? j.k_splits : 0;
     return rc;
 }
@@ -935,7 +938,7 @@ int pf_swiglu(const PfBuf& b, const void* w_gate, const void* w_up, int qtype, i
     PfJob j{};
     const int rc = pf_job(j, b, qtype, T, n_ff, cols, y, ld_y, w_gate, w_up, w_gate);
     if (rc != JINF_HIP_OK) return rc;
-    return pf_dispatch<kPfSwiGLU>(qtype, j, stream);
+    return pf_dispatch<kPfSwiGLU>(qtype, j, b, stream);
 }
 
 int pf_qkv(const PfBuf& b, const void* wq, const void* wk, const void* wv, int qtype, int T,
@@ -959,7 +962,7 @@ int pf_qkv(const PfBuf& b, const void* wq, const void* wk, const void* wv, int q
     j.kv_dim = kvd;
     j.head_dim = head_dim;
     j.max_ctx = max_ctx;
-    return pf_dispatch<kPfQKV>(qtype, j, stream);
+    return pf_dispatch<kPfQKV>(qtype, j, b, stream);
 }
 
 }  // namespace jinf

@@ -84,6 +84,50 @@ def test_row_widths(n_embd, heads, n_ff):
         check(e.logits(), decode(ref, toks), F32, f"{n_embd} / {n_ff}")
 
 
+def test_whole_rounds_and_a_split_tail():
+    """A gate / up product of 300 tiles: one round of 256 and 44 split in two."""
+    hp, W = mu.tiny_model(seed=15, n_layers=1, n_embd=512, n_heads=8, n_heads_kv=2, n_ff=12800,
+                          n_vocab=301, types=dict.fromkeys(MATS, Q4_0))
+    toks = tokens(260, 301, 15)
+    ref = oeng.Decoder(hp, W, max_context=272, kv_type=F16)
+    with jinf_amd.Engine(hp, mu.to_device(W), 272, F16) as e:
+        e.prefill(toks)
+        check(e.logits(), decode(ref, toks), F16, "260 tokens")
+
+
+def test_wide_rows_against_batched_steps():
+    """Residual adds of 264 tiles (one round, 8 split) and Q / K / V of 280 (24
+    split), 8448 columns: the logits of a 1000-token prompt against the same
+    prompt in batched steps of 50."""
+    hp, W = mu.tiny_model(seed=16, n_layers=1, n_embd=256, n_heads=2, n_heads_kv=2, n_ff=512,
+                          n_vocab=301)
+    n, kvd, ff = 8448, 256, 512
+    hp.update(n_embd=n, n_heads=66, n_heads_kv=2)
+    r = np.random.default_rng(16)
+
+    def q4_0(rows, cols, rms):
+        b = r.integers(0, 256, size=(rows, cols // 32, 18), dtype=np.uint8)
+        d = (r.uniform(0.5, 1.5, size=(rows, cols // 32)) * rms / 4.6).astype(np.float16)
+        b[:, :, :2] = d[..., None].view(np.uint8)
+        return b.reshape(rows, -1), Q4_0
+
+    W = {"token_embd.weight": q4_0(301, n, 1.0), "output.weight": q4_0(301, n, n ** -0.5),
+         "output_norm.weight": (mu.norm_weight(1, n, F32), F32)}
+    for name, rows, cols in (("attn_q", n, n), ("attn_k", kvd, n), ("attn_v", kvd, n),
+                             ("attn_output", n, n), ("ffn_gate", ff, n), ("ffn_up", ff, n),
+                             ("ffn_down", n, ff)):
+        W[f"blk.0.{name}.weight"] = q4_0(rows, cols, cols ** -0.5)
+    for name in ("attn_norm", "ffn_norm"):
+        W[f"blk.0.{name}.weight"] = (mu.norm_weight(2, n, F32), F32)
+    toks = tokens(1000, 301, 16)
+    with jinf_amd.Engine(hp, mu.to_device(W), 8, F16) as e, jinf_amd.Batch(e, 50, 1000, F16) as b:
+        b.prefill(0, toks)
+        got = b.logits()
+        for c in range(0, 1000, 50):
+            b.prefill(1, toks[c:c + 50])
+        check(got, b.logits().astype(np.float64), F16, "rows 950 .. 999")
+
+
 def test_two_chunks_and_a_later_prompt():
     """A prompt of two wide chunks, then another at a position inside the
     context (an attention tile starting past its first row)."""
