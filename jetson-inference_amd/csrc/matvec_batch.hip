@@ -528,10 +528,12 @@ __device__ __forceinline__ void mb_wait_w(int wave) {
 }
 
 template <int MT> constexpr int mb_occ() { return 2; }  // waves per SIMD the kernel is sized for
-// MERGE: split columns are merged in this launch.  An instantiation of its own
-// for residual adds and Q / K / V: the merge's code beside the partial stores,
-// even when not run, made the batch-32 step of the Q4_K_M layout 0.6% slower
-// (Q6_K down projection 27.3 -> 28.2 us).
+// MERGE: split columns are merged in this launch; an instantiation of its own
+// for residual adds and Q / K / V.  (The Q6_K down projection of the batch-32
+// step takes 26.6 to 28.2 us with the same loop, instruction for instruction,
+// depending on where the kernels of the library fall in the code object: 27.2
+// as one instantiation with the merge's code, 27.9 as two, 26.6 to 27.8 with
+// further instantiations or s_nop between.  No layout of it is pinned.)
 template <int QT, int MT, int EPI, int NT, int WV, int KSW, bool MERGE>
 __global__ __launch_bounds__(64 * WV, 4 * mb_occ<MT>() / WV) void matvec_batch_kernel(MbJob j, MbTheta<EPI> th) {
     constexpr int THREADS = 64 * WV;
