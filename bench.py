@@ -642,7 +642,7 @@ def batch_bench(args, torch, jinf_amd, spec):
     log(f"{args.steps} steps x {n_seq} sequences: {ms_step:.3f} ms per step, "
         f"{tok_s:.0f} tokens/s")
     # prompt processing: one sequence's 512-token prompt through
-    # jinf_hip_batch_prefill (chunks of n_seq tokens per step), after one
+    # jinf_hip_batch_prefill (steps of up to 1024 tokens), after one
     # untimed run
     import ctypes
     import numpy as np
@@ -661,7 +661,7 @@ def batch_bench(args, torch, jinf_amd, spec):
         if rc != 0:
             raise SystemExit(f"jinf_hip_batch_prefill failed ({rc})")
     if n_pf > 0:
-        log(f"prefill of {n_pf} tokens in chunks of {n_seq}: {pf_s * 1e3:.2f} ms, "
+        log(f"prefill of {n_pf} tokens: {pf_s * 1e3:.2f} ms, "
             f"{n_pf / pf_s:.0f} tokens/s")
     b.close()
     e.close()
@@ -831,8 +831,8 @@ def engine_bench(args, torch, jinf_amd):
     out = e.generate([], n_gen)
     gen_s = time.perf_counter() - t0
     log(f"token steps decoded in this run: {e.n_past}")
-    # a 512-token prompt: batched prefill (steps of 64 tokens on the batched
-    # GEMVs) against the token-by-token forward call, each from position 0
+    # a 512-token prompt: prefill (steps of up to 1024 tokens) against the
+    # token-by-token forward call, each from position 0
     n_pf = min(args.prompt_tokens, max_ctx)
     pf_toks = [int(t) for t in torch.randint(0, hp["n_vocab"], (max(n_pf, 1),), generator=g,
                                              device="cuda").cpu()]

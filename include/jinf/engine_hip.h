@@ -202,9 +202,10 @@ int  jinf_hip_batch_forward(jinf_hip_batch* b, const int32_t* tokens, const floa
 
 /* Prompt of sequence seq: decodes its n_tokens ids (each in [0, n_vocab)),
  * every projection running on a step's tokens at once (up to n_seq tokens in
- * a batched step; longer prompts in steps of up to 1024) and token i
- * attending to the sequence's positions up to its own, so the sequence ends where n_tokens forward steps of its own would
- * leave it (position advanced by n_tokens, next token the last token's
+ * a batched step, some prompts of up to 2 n_seq in two; longer ones in steps
+ * of up to 1024) and token i attending to the sequence's positions up to its
+ * own, so the sequence ends where n_tokens forward steps of its own would leave
+ * it (position advanced by n_tokens, next token the last token's
  * argmax); other sequences are untouched.  The logits of the prompt's last
  * m = (n_tokens - 1) mod n_seq + 1 tokens occupy rows 0 .. m - 1 of the
  * batch's logits; *logits (may be NULL) receives the device

@@ -268,7 +268,7 @@ int jinf_dequant_rows(void* out, int ld_out, const void* table, int qtype, int n
  * (kv head h / (n_heads / n_heads_kv)),
  *   out[s, h*hd:(h+1)*hd] = sum_t softmax_t(scale * q[s,h] . k[s,t,kv]) v[s,t,kv]
  * over t < lens[s] (clamped to [0, max_ctx]); a sequence with no position
- * gets zeros.  q and out are fp32 with row strides ld_q, ld_out (elements).
+ * gets zeros, one with a NaN score NaN.  q and out are fp32 with row strides ld_q, ld_out (elements).
  * Cache element (s, t, kv head j, dim d) is at s*ld_seq + t*ld_pos + j*hd + d
  * in k_cache / v_cache, of kv_type JINF_HIP_F32 or JINF_HIP_F16; ld_seq is at
  * least max_ctx * ld_pos when n_seq > 1, or 0 (every row reads the same
@@ -299,8 +299,9 @@ size_t jinf_attention_workspace_bytes(int n_seq, int n_heads, int head_dim, int 
 /* jinf_attention_decode without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  Same
- * arguments, results and kernels as jinf_attention_decode with a workspace
- * (bit-identical outputs); the split contexts keep their merge counters and
+ * arguments, results and kernels as jinf_attention_decode with a workspace for
+ * an fp16 cache and without one for an fp32 cache (bit-identical outputs); the
+ * split contexts keep their merge counters and
  * chunk records in a library-owned scratch array in device memory instead:
  * 256 bytes of counters plus 8 MiB of records, one copy per device, held until
  * the process ends.  Nothing is allocated or freed by the call.

@@ -253,8 +253,8 @@ class Batch:
         return p.value
 
     def prefill(self, seq, tokens):
-        """Sequence seq's prompt in chunks of up to n_seq tokens per step;
-        returns the last token's logits, fp32 [n_vocab] (host copy)."""
+        """Sequence seq's prompt in steps of up to 1024 tokens (up to n_seq
+        tokens: one batched step); returns the last token's logits, fp32 [n_vocab] (host copy)."""
         t = np.ascontiguousarray(np.asarray(tokens, dtype=np.int32).reshape(-1))
         p = ctypes.c_void_p()
         _check("jinf_hip_batch_prefill",

@@ -276,13 +276,14 @@ def test_prefill_wide_chunks(dev):
 
 @pytest.mark.parametrize("name", ["mixed", "hd128-gqa4-f16embd"])
 def test_long_prefill_splits_attention_contexts(dev, name):
-    """A 330-token prompt through the batch decoder's prefill (chunks of 64
-    tokens, one per sequence slot, sharing one KV region) at max_context 512
-    with an fp16 cache: contexts past 256 positions are split and merged by
-    the separate merge launch (64 rows x 2 head groups in "mixed") or inside
-    the attention launch (the 10-token last chunk; 64 x 1 groups in the
-    other model).  The last token's logits and the next step of that
-    sequence equal the oracle's loop."""
+    """A 330-token prompt through the batch decoder's prefill (one wide step)
+    at max_context 512 with an fp16 cache, then a decode step of 64 rows, one
+    of them over a context past 256 positions: split and merged by the
+    separate merge launch (64 rows x 2 head groups in "mixed") or inside the
+    attention launch (64 x 1 groups in the other model).  The last token's
+    logits and that step equal the oracle's loop.  (Batched steps and wide
+    prompts whose own contexts are split: test_gpu_attention_merge.py,
+    test_gpu_prefill_wide.py.)"""
     n_seq, max_ctx = 64, 512
     say(f"batch prefill of 330 tokens, {name}, max_context {max_ctx}, kv f16")
     hp, W = mu.tiny_model(seed=66, n_vocab=350, **MODELS[name])

@@ -296,12 +296,11 @@ def test_gguf_missing_tensor(dev, tmp_path):
 @pytest.mark.parametrize("name", ["mixed", "hd128-gqa4"])
 def test_long_prefill_splits_attention_contexts(dev, name):
     """A 330-token prompt through prefill at max_context 512 with an fp16 KV
-    cache: the attention of every 64-token step runs over contexts past one
-    256-position chunk, so its split contexts are merged -- by the separate
-    merge launch when the step has 128 or more (row, head group) pairs
-    ("mixed": 64 rows x 2 groups), inside the attention launch otherwise
-    (the 10-token last step; "hd128-gqa4": 64 rows x 1 group).  The last
-    token's logits and the next decode step equal the oracle's loop."""
+    cache, in one wide step; the next decode step's attention runs over a
+    context past one 256-position chunk, split and merged inside the launch.
+    The last token's logits and that step equal the oracle's loop.  (Batched
+    steps and wide prompts whose own contexts are split:
+    test_gpu_attention_merge.py, test_gpu_prefill_wide.py.)"""
     max_ctx = 512
     say(f"engine prefill of 330 tokens, {name}, max_context {max_ctx}, kv f16")
     hp, W = mu.tiny_model(seed=24, **MODELS[name])
