@@ -352,7 +352,7 @@ int bat_wide_create(jinf_hip_batch* b) {
     const size_t o_attn = take_b(rows * b->q_dim * 4), o_ff = take_b(rows * nff * 4);
     const size_t o_up = take_b(split_ffn ? rows * nff * 4 : 0);
     const size_t o_rec = take_b(pf_rec_bytes(R, (int)std::max(n, nff)));
-    const size_t o_inv = take_b(rows * (std::max(n, nff) / 256) * 4);
+    const size_t o_xs = take_b(rows * (std::max(n, nff) / 256) * 8);
     const size_t o_cs = take_b(rows * (size_t)b->head_dim / 2 * 8);
     const size_t o_part = take_b(pf_part_bytes()), o_rows = take_b(3 * rows * 4);
     const RelaxedCapture relaxed;
@@ -368,7 +368,7 @@ int bat_wide_create(jinf_hip_batch* b) {
     b->w_rows = reinterpret_cast<int32_t*>(b->wide + o_rows);
     b->pf.rows = R;
     b->pf.rec = reinterpret_cast<uint8_t*>(b->wide + o_rec);
-    b->pf.inv_s = f(o_inv);
+    b->pf.xs = f(o_xs);
     b->pf.cs = reinterpret_cast<float2*>(b->wide + o_cs);
     b->pf.part = f(o_part);
     b->pf.part_bytes = pf_part_bytes();

@@ -28,15 +28,19 @@
 // tokens the same products take 296 and 860 us.
 //
 // Sums: MFMA chains of one block (hi products first: the lo ones added first
-// measured a 35% larger error), scaled into a first-level sum of a slab (Q6_K,
-// with twice the blocks: half a slab), those times the slab's 1 / s into a
-// second.  Relative error of a layer's logits against fp64, batched steps ->
-// here (1024 to 4096 columns, 72 and 300 tokens): Q4_0 and Q8_0 1.6-2.0e-7 ->
-// 0.93-1.00 of it, Q6_K 1.6-2.1e-7 -> 0.87-0.99, Q4_K 3.7-4.2e-7 -> 0.45-0.47.
-// (First-level sums of two slabs under one scale per row: 1 to 2% faster
-// (Q6_K 5%), but Q6_K up to 1.07, Q4_0 1.02, and small columns of the output
-// and down projections' inputs beside ones 2^22 times larger three to four
-// times the error; the batched steps scale each column split by itself.)
+// measured a 35% larger error), scaled into a first-level sum of a slab, those
+// times the slab's 1 / s into a second; except in gate / up, and in residual
+// adds of Q6_K, what the second level's additions round away is carried along
+// (Q6_K there sums half slabs, as it has twice the blocks).  Error against
+// fp64 relative to that of batched steps (a layer's logits, fp32 cache, 72, 300
+// and 1000 tokens, 1024 to 4096 columns): Q4_0 and Q8_0 0.92-1.00, Q4_K
+// 0.45-0.54, Q6_K 0.87-1.01; 1000 tokens of 4096 / 14336 with an fp16 cache
+// 0.88-0.96 (Q4_K 0.59).  Tried: first-level sums of two slabs under one scale
+// per row, 3 to 4% faster at 1000 tokens (Q6_K 6%), but up to 1.07, and small
+// columns of the output and down projections' inputs beside ones 2^22 times
+// larger three to four times the error, as the batched steps scale each column
+// split by itself; without the carry, 2 to 2.5% faster, but 1.01 and with the
+// fp16 cache 1.04-1.16 at 1000 tokens of 4096 / 14336.
 // Q4_K's minimum goes in through its codes' centre: coefficient and 32-column
 // sums of x as fp16 hi + lo (the batched steps': fp32), which the centred
 // codes' smaller terms more than make up for (medians with every minimum
@@ -88,8 +92,7 @@ struct PfJob {
     int accum;
     int64_t row_bytes;
     const uint8_t* rec;
-    const float* inv_s;    // [n_slabs][ld_inv]
-    int ld_inv;
+    const float* xs;
     float* y;
     int ld_y;
     float* part;           // partial sums of split tiles: [k_splits][T][rows] when
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(256) void pf_merge_kernel(float* __restrict__ x, in
 // tokens of 4096 / 14336 take the same either way (8.70 ms for 8 layers).  With
 // a scale per slab, half a wave's maximum, a row without a norm needs no
 // barrier: 28.5 -> 27.6 us for 1000 tokens of 14336 columns, 17.7 -> 16.8 of
-// 4096.  A
+// 4096 (with a norm).  A
 // token owns 16 bytes of each 512-byte run of a record, so the 8 tokens of a
 // 128-byte line go to workgroups of one XCD, whose L2 joins them.  Tokens
 // past T, up to the next whole tile, are zeros.
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(256) void pf_prepare_kernel(float* __restrict__ x, 
                                                          int k, int64_t stride,
                                                          const void* __restrict__ norm_w,
                                                          int norm_f16, float eps,
-                                                         float* __restrict__ inv_s, int ld_inv,
+                                                         float* __restrict__ xs,
                                                          uint8_t* __restrict__ rec) {
     __shared__ double red[4];
     const int xcd = blockIdx.x & 7, ix = blockIdx.x >> 3;
@@ -226,7 +229,14 @@ __global__ __launch_bounds__(256) void pf_prepare_kernel(float* __restrict__ x, 
         m = fmaxf(m, __shfl_xor(m, 16, kWave));
         const int ex = mb_scale_exp(m);
         const float sc = ldexpf(1.0f, 15 - ex);
-        if ((g & 31) == 0) inv_s[(int64_t)(g >> 5) * ld_inv + t] = ldexpf(1.0f, ex - 15);
+        if ((g & 31) == 0) {
+            // (s above 2^30 is written as 0: it only scales a carried rounding
+            // error, which that slab then goes without, into acc's units, and
+            // has to stay in range)
+            float* p = xs + ((int64_t)(t / kPfTile) * (ng / 32) + (g >> 5)) * (2 * kPfTile) + t % kPfTile;
+            p[0] = ldexpf(1.0f, ex - 15);
+            p[kPfTile] = sc <= 0x1p30f ? sc : 0.0f;
+        }
         // columns in the order (0, 4, 1, 5, 2, 6, 3, 7); the sums are of the
         // split values
         uint32_t hw[4], lw[4];
@@ -381,7 +391,7 @@ struct PfShape {
     static constexpr int DB = NSC * 64 * NW * 4;
     static constexpr int CB = QT == kQ4_K ? 64 * NW * 36 : 0;  // hi and lo coefficients, factor
     static constexpr int SB = QT == kQ4_K ? TILES * 1024 : 0;
-    static constexpr int IB = 1024;  // a slab's 1 / s of the 128 tokens (twice)
+    static constexpr int IB = 2 * kPfTile * 4;  // a slab's 1 / s and s of the tokens
     static constexpr int LDS = 2 * (XB + WB + DB + CB + SB + IB);
     static_assert(32 * TILES == kPfTile && LDS <= 160 * 1024, "shape");
 };
@@ -416,6 +426,8 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
     const int mtile = tile % j.n_mt, nt_ = tile / j.n_mt;
     const int s0 = whole ? 0 : split * j.slabs_per_split;
     const int s1 = whole ? j.n_slabs : min(j.n_slabs, s0 + j.slabs_per_split);
+
+    const int st0 = 4 * s0, st1 = 4 * s1;  // stages
 
     uint8_t* const xbuf = pf_lds;
     uint8_t* const wbuf = xbuf + 2 * S::XB;
@@ -480,8 +492,8 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
         *reinterpret_cast<mb_h8*>(wdst + b * S::WB + (o >> 1) * 1024 + (o & 1) * 512) =
             pf_decode8<QT>(raw, o, wg);
     };
-    // x fragments of stage st (and, in its slab's first, the tokens' 1 / s
-    // and, Q4_K, the slab's sums)
+    // x fragments of stage st, the scales of the first and, a stage before
+    // each slab's end, of the next slab, and (Q4_K) the slab's sums in its first
     auto issue_x = [&](int st) {
         const int slab = st >> 2;
         uint8_t* dst = xbuf + (st & 1) * S::XB;
@@ -493,10 +505,12 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
                             (2 * KST * (st & 3) + r) * 1024,
                         16u * lane, dst + a * 1024);
         }
-        if ((st & 3) == 0 && wave == 7)
-            pf_lds_load(reinterpret_cast<const uint8_t*>(j.inv_s + (int64_t)slab * j.ld_inv +
-                                                         mtile * kPfTile),
-                        16u * (lane & 31), ibuf + (slab & 1) * S::IB);
+        if (wave == 7 && (st == st0 || ((st & 3) == 3 && st + 1 < st1))) {
+            const int sl = st == st0 ? slab : slab + 1;
+            pf_lds_load(reinterpret_cast<const uint8_t*>(j.xs + ((int64_t)mtile * j.n_slabs + sl) *
+                                                                    (2 * kPfTile)),
+                        16u * lane, ibuf + (sl & 1) * S::IB);
+        }
         if constexpr (QT == kQ4_K) {
             if ((st & 3) == 0 && wave < TILES)
                 pf_lds_load(j.rec + ((int64_t)(mtile * TILES + wave) * j.n_slabs + slab) * kPfRec + 32768,
@@ -505,11 +519,18 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
     };
 
     // Two-level sums: acc takes the blocks of kFlush stages, in units of x s,
-    // then is scaled by the slab's 1 / s, added to sum and cleared.  A value
-    // is rounded by at most 8 (Q4_0, Q8_0; Q6_K, of 16-column blocks) or 9
-    // (Q4_K) block FMAs of a first-level sum and by the row's 2 or 1 flushes
-    // per slab, besides the matrix-core chains' own roundings.
-    constexpr int kFlush = QT == kQ6_K ? 2 : 4;
+    // then is scaled by the slab's 1 / s, added to sum and cleared.  kCarry:
+    // what that addition rounds away starts the next acc instead, in its slab's
+    // units.  So a value is rounded by at most 8 (Q4_0, Q8_0; Q6_K without a
+    // carry, in 16-column blocks), 9 (Q4_K) or 16 (Q6_K) block FMAs of a
+    // first-level sum, and then once, or without a carry by the row's 1 (Q6_K
+    // 2) additions per slab, besides the matrix-core chains' own roundings.  (A
+    // sum beyond fp32's range ends as NaN with a carry, as infinity without.)
+    // The carry costs 4 instructions a value and slab instead of 2; gate / up,
+    // 43% of the time, goes without: its second level has 16 additions at 4096
+    // columns where the batched steps chain 32 blocks.
+    constexpr bool kCarry = EPI == kPfQKV || (EPI == kPfAdd && QT != kQ6_K);
+    constexpr int kFlush = QT == kQ6_K && !kCarry ? 2 : 4;
     mb_f16 acc[2][MT], sum[2][MT];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -518,22 +539,29 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
     auto flush = [&](int slab) {
         const float* iv = reinterpret_cast<const float*>(ibuf + (slab & 1) * S::IB) +
                           32 * mw * MT + 4 * h;
+        const float* nx = reinterpret_cast<const float*>(ibuf + ((slab & 1) ^ 1) * S::IB) +
+                          kPfTile + 32 * mw * MT + 4 * h;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float4 w = *reinterpret_cast<const float4*>(iv + 32 * mt + 8 * q);
                 const float f[4] = {w.x, w.y, w.z, w.w};
+                float g[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (kCarry) {
+                    const float4 u = *reinterpret_cast<const float4*>(nx + 32 * mt + 8 * q);
+                    g[0] = u.x; g[1] = u.y; g[2] = u.z; g[3] = u.w;
+                }
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        sum[i][mt][4 * q + e] = fmaf(acc[i][mt][4 * q + e], f[e], sum[i][mt][4 * q + e]);
+                    for (int e = 0; e < 4; ++e) {
+                        const float a = acc[i][mt][4 * q + e], old = sum[i][mt][4 * q + e];
+                        const float t = fmaf(a, f[e], old);
+                        sum[i][mt][4 * q + e] = t;
+                        acc[i][mt][4 * q + e] = kCarry ? fmaf(a, f[e], old - t) * g[e] : 0.0f;
+                    }
             }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[i][mt] = mb_f16{};
     };
     // Q4_K: the finished slab's coefficient times sum products
     auto corrections = [&](int slab) {
@@ -561,7 +589,6 @@ __global__ __launch_bounds__(512, 2) void pf_matmul_kernel(PfJob j) {
     // Stage st computes on x and weight fragments in buffers st & 1, while x
     // of st + 1 is loaded, the weights of st + 1 (loaded during st - 1) are
     // decoded into the other buffer, and those of st + 2 are loaded.
-    const int st0 = 4 * s0, st1 = 4 * s1;
     issue_x(st0);
     raw = pf_load_raw<QT>(wrow, 2 * st0 + wblk);
 #pragma unroll
@@ -868,8 +895,7 @@ int pf_job(PfJob& j, const PfBuf& b, int qtype, int T, int rows, int cols, float
     j.seg_end[0] = j.seg_end[1] = j.seg_end[2] = rows;
     j.row_bytes = (int64_t)(cols / e) * bytes;
     j.rec = b.rec;
-    j.inv_s = b.inv_s;
-    j.ld_inv = b.rows;
+    j.xs = b.xs;
     j.y = y;
     j.ld_y = ld_y;
     j.part = b.part;
@@ -906,7 +932,7 @@ int pf_prepare(const PfBuf& b, float* x, int ld_x, int T, int cols, const void* 
                            : pf_prepare_kernel<16>;
     const int rc = launch(kern, dim3(tokens), dim3(256), 0, stream, x, ld_x, cols, T,
                           static_cast<const float*>(b.part), k, (int64_t)T * cols, norm_w, f16, eps,
-                          b.inv_s, b.rows, b.rec);
+                          b.xs, b.rec);
     if (rc == JINF_HIP_OK && pend) pend->k = 0;
     return rc;
 }

@@ -17,7 +17,7 @@ constexpr int kPfTile = 128;
 struct PfBuf {
     int rows = 0;            // tokens they hold (a multiple of kPfTile)
     uint8_t* rec = nullptr;  // x as matrix-core fragments
-    float* inv_s = nullptr;  // [slabs][rows] 1 / s of the prepared x
+    float* xs = nullptr;     // the prepared x's scales: [128-token tile][slab][1 / s, s][128]
     float2* cs = nullptr;    // [rows][head_dim / 2] RoPE cos, sin
     float* part = nullptr;   // partial sums of split columns
     size_t part_bytes = 0;
